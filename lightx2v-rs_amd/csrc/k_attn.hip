@@ -5,22 +5,34 @@
 //   out[q, h*d + j] = sum_k softmax_k(q.k / sqrt(d), masked) v[k, j]
 //   q [heads, sq, d], k / v [heads, sk, d], mask [sq, sk] (1 = allowed)
 //
-// k_attn_mfma (d = 64 or 128): one workgroup per (head, 128 queries), four
+// k_attn_mfma (d = 64 or 128): one workgroup per (head, 256 queries), eight
 // waves of 32 queries, keys in tiles of 64 through LDS, online softmax
 // (running max and sum per query, exp2 with log2(e)/sqrt(d) folded in).
 // Each wave computes S^T = K Q^T with v_mfma_f32_32x32x16_bf16 (K is the A
 // operand, Q the B operand held in registers), so a lane owns one query and
-// 32 of its keys: the row max and sum take one cross-lane step.  P^T stays
-// in the registers it was computed in and is the B operand of O^T = V^T P^T;
-// the keys of each 16-key MFMA step are taken in the order the S^T layout
-// left them in the lane (4 keys of group g, then 4 of group g + 1), and V^T
-// is read from LDS in that same order, so no transpose of P is needed.
+// 32 of its keys: the row max takes one cross-lane step, the row sum one at
+// the very end.  P^T stays in the registers it was computed in and is the B
+// operand of O^T = V^T P^T; the keys of each 16-key MFMA step are taken in
+// the order the S^T layout left them in the lane (4 keys of group g, then 4
+// of group g + 2), and V^T's fragments come out of LDS in that same order by
+// the transposing read, so neither P nor V is transposed by instructions.
 // A per-(query tile, key tile) mask summary skips fully masked tiles and
-// reads mask bytes only in mixed ones.
+// reads mask words only in mixed ones.
+//
+// What bounds it: the matrix cores and the vector ALU of a SIMD together.  A
+// 64-key tile is 2 x 1024 cycles of MFMA per SIMD (two waves) and 2 x about
+// 155 VALU instructions (32 of them exponentials) that overlap the MFMAs only
+// in part.  Dealing MFMAs, LDS reads and softmax out step by step took the
+// 12 x 128, 4680 x 6240 frame-causal call from 204 to 152 us (1.45 us per
+// tile; with every CU loaded that is 1.4 PFLOP/s, what a large bf16 matrix
+// product reaches here), and 4680 x 18720 over the cache from 600 to 470.
+// Row sums or maxima left out, LDS reads, loads or exponentials left out of
+// timing copies: 1 to 8% each; other fragment depths, barrier places and wave
+// priorities: within 1%.
 //
 // k_attn_rows: any d <= 256, one wave per (head, query), keys one at a
 // time -- the correctness path for other head sizes.
-#include "device_common.hpp"
+#include "gemm_common.hpp"
 #include "runtime.hpp"
 
 namespace lx2v {
@@ -47,22 +59,45 @@ __device__ __forceinline__ u32x4 ld8_bf16(const void *p, size_t i) {
     }
 }
 
+// Key tiles are staged in LDS as they are, [key][d] rows of bf16: K in a ring
+// of three slots, V in two, 16 bytes a lane straight from global memory (f32
+// inputs: through registers, rounded).
+//
+// K: 1 KB blocks, what one wave's load writes: KB rows, 64 bytes of padding
+// after each block, and chunk c of row r at chunk c ^ kswz(r) (two bits).  The
+// 16 rows a fragment read touches at once then fall in distinct banks (four
+// chunk positions x four paddings, or with D = 64 four positions x two half
+// rows x two paddings), and a lane's chunk 2 s + hf needs two addresses in
+// all (s even, s odd) beside immediates.
+//
+// V: no padding; 64-byte segment g of row r at segment g ^ vswz(r).  V^T's
+// fragments come from the transposing read (ds_read_b64_tr_b16: within each
+// 16 lanes, lane 4 j + r gives the address of 4 d of key j and lane i
+// receives d i of keys 0..3), whose 32 lanes read 64 bytes of four
+// consecutive rows: with the swizzle these are all 64 banks.
+template <int D>
+struct AttnLds {
+    static constexpr int CH = D / 8;            // 16-byte chunks per row
+    static constexpr int KB = 64 / CH;          // rows per block
+    static constexpr int KBS = 1024 + 64;       // bytes per K block
+    static constexpr int KSZ = AK / KB * KBS, VSZ = AK * D * 2;
+    static constexpr int V0 = 0, K0 = 2 * VSZ, BYTES = K0 + 3 * KSZ;
+    static __device__ __forceinline__ int kswz(int r) { return (r / (KB / 4)) & 3; }
+    static __device__ __forceinline__ int vswz(int r) { return (r / (KB / 4)) & (D / 32 - 1); }
+};
+
 template <int D, int DT, int ODT>
 __global__ __launch_bounds__(AT) void k_attn_mfma(const void *__restrict__ Q, const void *__restrict__ K,
                                                   const void *__restrict__ V, int heads, int sq, int sk, int kvs,
                                                   const uint8_t *__restrict__ tiles, const uint32_t *__restrict__ mbits,
                                                   float c, void *__restrict__ out, uint8_t *__restrict__ omx,
                                                   int omx_rows, float *__restrict__ part, int nsplit) {
-    constexpr int KSTR = D * 2 + 16;   // bytes per K row in LDS (padded: conflict-free fragment reads)
-    // bytes per V^T row (one d, 64 keys): 9 16-byte chunks, so the 16-byte
-    // fragment reads of 16 consecutive rows fall in distinct bank groups
-    constexpr int VSTR = AK * 2 + 16;
+    using L = AttnLds<D>;
     constexpr int QS = D / 16;         // 16-wide d steps of S^T
     constexpr int DB = D / 32;         // 32-row d blocks of O^T
-    constexpr int KN = AK * D / 8, VN = AK * D / 16, KI = (KN + AT - 1) / AT, VI = (VN + AT - 1) / AT;
-    constexpr int KSZ = AK * KSTR, VSZ = D * VSTR;
-    // K of tiles t + 1 and t + 2, V of tiles t and t + 1: [K0 K1 V0 V1].
-    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * (KSZ + VSZ)];
+    constexpr int KI = AK * D / 8 / AT;  // 16-byte chunks of a K or V tile per thread
+    static_assert(KI * AT * 8 == AK * D, "whole rounds");
+    __shared__ __attribute__((aligned(16))) uint8_t lds[L::BYTES];
 
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, l32 = lane & 31, hf = lane >> 5;
     // XCD-aware order: workgroups b, b + 8, ... run on one XCD, so give each
@@ -136,163 +171,140 @@ __global__ __launch_bounds__(AT) void k_attn_mfma(const void *__restrict__ Q, co
     for (int s = 0; s < QS; s++)
         qf[s] = __builtin_bit_cast(bf16x8, qin ? ld8_bf16<DT>(Q, qbase + 16 * s + 8 * hf) : (u32x4){});
 
+    // This query tile's key tiles with an allowed pair, in order, as key tile
+    // | state << 14 (state 1: every pair allowed, 2: mixed), compacted by
+    // wave 0 with ballots.  Without a mask, or past TROW tiles, entry i is
+    // tile i itself (all allowed, or read as mixed).
+    __shared__ uint16_t list[TROW];
+    __shared__ int nlist;
+    const bool tlds = tiles && nkt <= TROW;
+    if (tlds && wv == 0) {
+        int total = 0;
+        for (int base = 0; base < nkt; base += 64) {
+            const int t = base + lane;
+            const int st = t < nkt ? tiles[(size_t)qt * nkt + t] : 0;
+            const uint64_t bal = __ballot(st != 0);
+            if (st) list[total + __popcll(bal & ((1ull << lane) - 1ull))] = (uint16_t)(t | st << 14);
+            total += __popcll(bal);
+        }
+        if (lane == 0) nlist = total;
+    }
     // Q in registers before the loop: otherwise the first use of qf in every
     // iteration waits for all loads in flight, the next tile's included.
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    __syncthreads();
+    const int nall = tlds ? nlist : nkt;
+    // This workgroup's entries [i0, i0 + n): all, or in split mode those from
+    // the floor(p n / S)-th to the floor((p + 1) n / S)-th (piece p).
+    const int i0 = split ? (int)((long long)piece * nall / nsplit) : 0;
+    const int n = (split ? (int)((long long)(piece + 1) * nall / nsplit) : nall) - i0;
+    const int whole = tiles ? 2 : 1;  // the state of a tile that is not listed
+    // key tile | state << 24; -1 past the last
+    auto entry = [&](int i) -> int {
+        if (i >= n) return -1;
+        if (!tlds) return (i0 + i) | whole << 24;
+        const int v = list[i0 + i];
+        return (v & 0x3FFF) | (v >> 14) << 24;
+    };
+    auto tile_of = [](int e) { return e & 0xFFFFFF; };
+    auto state_of = [](int e) { return e >> 24; };
 
     f32x16 o[DB];
 #pragma unroll
     for (int b = 0; b < DB; b++) o[b] = (f32x16){};
-    float m = -INFINITY, lsum = 0.0f;  // running max (log2 domain, scaled) and sum
+    float m = -INFINITY, lsum = 0.0f;  // running max (log2 domain, scaled); sum over this lane's own keys
 
-    // This query tile's row of the mask summary, staged in LDS (a global
-    // load per tile would cost a memory latency per tile); rows longer than
-    // the stage skip the summary: every tile is then read as mixed.
-    __shared__ uint8_t trow[TROW];
-    const bool tlds = tiles && nkt <= TROW;
-    if (tlds)
-        for (int i = tid; i < nkt; i += AT) trow[i] = tiles[(size_t)qt * nkt + i];
-    __syncthreads();
-    auto tstate = [&](int kt) -> int { return !tiles ? 1 : (tlds ? (int)trow[kt] : 2); };
-    // This workgroup's key tiles [klo, khi): all of them, or in split mode,
-    // of the n tiles with an allowed pair, those after the floor(p n / S)-th
-    // up to and including the floor((p + 1) n / S)-th (piece p; the last
-    // piece runs to the end).  Wave 0 counts with ballots.
-    int klo = 0, khi = nkt;
-    if (split) {
-        __shared__ int scut[2];
-        if (wv == 0) {
-            int total = 0;
-            for (int base = 0; base < nkt; base += 64) {
-                const int t = base + lane;
-                total += __popcll(__ballot(t < nkt && tstate(t) != 0));
-            }
-            // cut(c): the tile after the c-th allowed one (cut(0) = 0)
-            const int c0 = (int)((long long)piece * total / nsplit), c1 = (int)((long long)(piece + 1) * total / nsplit);
-            int cut0 = 0, cut1 = 0, acc = 0;
-            for (int base = 0; base < nkt; base += 64) {
-                const int t = base + lane;
-                const bool al = t < nkt && tstate(t) != 0;
-                const uint64_t bal = __ballot(al);
-                const int cnt = __popcll(bal);
-                const uint64_t upto = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);
-                const int upto_cnt = acc + __popcll(bal & upto);
-                if (c0 > acc && c0 <= acc + cnt)
-                    cut0 = base + __ffsll((long long)__ballot(al && upto_cnt == c0));
-                if (c1 > acc && c1 <= acc + cnt)
-                    cut1 = base + __ffsll((long long)__ballot(al && upto_cnt == c1));
-                acc += cnt;
-            }
-            if (lane == 0) {
-                scut[0] = cut0;
-                scut[1] = piece == nsplit - 1 ? nkt : cut1;
-            }
-        }
-        __syncthreads();
-        klo = scut[0];
-        khi = scut[1];
-    }
-    // The next key tile at or after kt with an allowed pair (uniform).
-    auto next_tile = [&](int kt) {
-        while (kt < khi && tstate(kt) == 0) kt++;
-        return kt;
-    };
-
-    // Tiles from global memory into registers: K as 16-byte chunks (key,
-    // chunk), V as chunk pairs of two consecutive keys (for V^T).  Buffer
-    // loads: keys past sk (and unused lanes, offset kOob) read zero, and
-    // every load is issued, so waits can count the loads in flight.
+    // Global loads through buffer descriptors: keys past sk, and every
+    // offset of a tile past the last (kOob), read zero, so the loads need no
+    // branch.  K of bf16 inputs goes straight into LDS; f32 K is loaded to
+    // registers, rounded and stored at the end of the same iteration.
     constexpr uint32_t ES = DT == LX2V_DTYPE_BF16 ? 2 : 4;
+    constexpr int R8 = ES / 2;  // 16-byte loads per 8 elements
     const auto ksrc = make_rsrc((const uint8_t *)K + kvbase * ES, (uint32_t)sk * D * ES);
     const auto vsrc = make_rsrc((const uint8_t *)V + kvbase * ES, (uint32_t)sk * D * ES);
-    auto ld8 = [&](__amdgpu_buffer_rsrc_t r, uint32_t off, bool in) -> u32x4 {
-        if constexpr (DT == LX2V_DTYPE_BF16) {
-            return buffer_load_x4(r, in ? off * 2 : kOob);
-        } else {
-            const f32x4 a = __builtin_bit_cast(f32x4, buffer_load_x4(r, in ? off * 4 : kOob));
-            const f32x4 b = __builtin_bit_cast(f32x4, buffer_load_x4(r, in ? off * 4 + 16 : kOob));
-            return (u32x4){pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w), pack_bf16x2(b.x, b.y), pack_bf16x2(b.z, b.w)};
-        }
-    };
-    u32x4 kr[KI], va[VI], vb[VI];
-    uint32_t mwn[2];  // mask bits of the V tile loaded last (mixed tiles; kOob reads 0 otherwise)
     const uint32_t nw = ((uint32_t)sk + 31) / 32;
     const auto msrc = make_rsrc(mbits, mbits ? (uint32_t)sq * nw * 4 : 0u);
-    auto gload_k = [&](int kt) {
-        const uint32_t k0 = (uint32_t)kt * AK;
+    const uint32_t moff = qin ? (uint32_t)q * nw * 4 : kOob;
+    // Round it of a tile: this thread's chunk is row / position of chunk it AT
+    // + tid, loaded from the swizzled place.
+    uint32_t koff[KI], voff[KI];
 #pragma unroll
-        for (int it = 0; it < KI; it++) {
-            const int idx = it * AT + tid, key = idx / (D / 8), ch = idx % (D / 8);
-            kr[it] = ld8(ksrc, (k0 + key) * D + 8 * ch, idx < KN && kt < khi);
-        }
+    for (int it = 0; it < KI; it++) {
+        const int ck = it * AT + tid, row = ck / L::CH, pos = ck % L::CH;
+        koff[it] = (uint32_t)(row * D + 8 * (pos ^ L::kswz(row))) * ES;
+        voff[it] = (uint32_t)(row * D + 8 * (pos ^ (4 * L::vswz(row)))) * ES;
+    }
+    const uint32_t kdst = __builtin_amdgcn_readfirstlane(lds_addr(lds) + (uint32_t)(L::K0 + wv * L::KBS));
+    const uint32_t vdst = __builtin_amdgcn_readfirstlane(lds_addr(lds) + (uint32_t)(L::V0 + wv * 1024));
+    // Fragment addresses.  K: chunk (2 s + hf) of row 32 j + l32.  V: for d
+    // block b and keys k0 .. k0 + 3, row k0 + j of d 32 b + 16 (group & 1) + 4 r
+    // (this lane being 4 j + r of its 16-lane group).
+    const uint8_t *const kfr = lds + L::K0 + (l32 / L::KB) * L::KBS + (l32 % L::KB) * (D * 2);
+    const uint8_t *const kfr2[2] = {kfr + ((hf ^ L::kswz(l32)) * 16), kfr + (((2 + hf) ^ L::kswz(l32)) * 16)};
+    const uint8_t *vfr[DB];
+#pragma unroll
+    for (int b = 0; b < DB; b++) {
+        const int j = (lane / 4) % 4, r = lane % 4, row = 4 * hf + j;
+        vfr[b] = lds + L::V0 + row * (D * 2) + ((b ^ L::vswz(row)) * 64) + 32 * ((lane / 16) & 1) + 8 * r;
+    }
+
+    u32x4 kr[KI][R8], vr[KI][R8];  // f32 inputs only
+    uint32_t mwn[2] = {0u, 0u};    // mask words of the next tile (mixed tiles; kOob reads 0 otherwise)
+    // e < 0: past the last tile (the offset's top bit then puts it out of range).
+    auto oob = [](bool in) -> uint32_t { return in ? 0u : kOob; };
+    auto raw8 = [&](__amdgpu_buffer_rsrc_t r, uint32_t off, u32x4 *d) {
+#pragma unroll
+        for (int h = 0; h < R8; h++) d[h] = buffer_load_x4(r, off + 16 * h);
     };
-    auto gload_v = [&](int kt) {
-        const uint32_t k0 = (uint32_t)kt * AK;
-        const bool mixed = kt < khi && tstate(kt) == 2 && qin;
-#pragma unroll
-        for (int kb = 0; kb < 2; kb++)
-            mwn[kb] = buffer_load_x1(msrc, mixed ? ((uint32_t)q * nw + k0 / 32 + (uint32_t)kb) * 4 : kOob);
-        // V item idx: key pair idx % 32 (keys 2 p, 2 p + 1), chunk idx / 32 --
-        // consecutive lanes take consecutive key pairs, so the transposed
-        // stores below hit consecutive LDS words
-#pragma unroll
-        for (int it = 0; it < VI; it++) {
-            const int idx = it * AT + tid, key = 2 * (idx % (AK / 2)), ch = idx / (AK / 2);
-            va[it] = ld8(vsrc, (k0 + key) * D + 8 * ch, idx < VN && kt < khi);
-            vb[it] = ld8(vsrc, (k0 + key + 1) * D + 8 * ch, idx < VN && kt < khi);
-        }
+    auto bf8 = [&](const u32x4 *d) -> u32x4 {
+        const f32x4 a = __builtin_bit_cast(f32x4, d[0]), b = __builtin_bit_cast(f32x4, d[R8 - 1]);
+        return (u32x4){pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w), pack_bf16x2(b.x, b.y), pack_bf16x2(b.z, b.w)};
     };
-    // Registers into LDS: K rows; V transposed (one d per row).
-    auto lstore_k = [&](int buf) {
-        uint8_t *ks = lds + buf * KSZ;
-#pragma unroll
-        for (int it = 0; it < KI; it++) {
-            const int idx = it * AT + tid, key = idx / (D / 8), ch = idx % (D / 8);
-            if (idx < KN) *(u32x4 *)(ks + key * KSTR + ch * 16) = kr[it];
-        }
+    auto load_k = [&](int it, int slot, int e) {
+        const uint32_t off = (koff[it] + (uint32_t)tile_of(e) * (AK * D * ES)) | oob(e >= 0);
+        if constexpr (DT == LX2V_DTYPE_BF16)
+            dma16_at(ksrc, kdst + slot * L::KSZ + it * (AT / 64) * L::KBS, off);
+        else
+            raw8(ksrc, off, kr[it]);
     };
-    // V^T key order: bits 2 and 3 of the key swapped, so that the 8 keys a
-    // lane feeds one 16-key MFMA step (4 of group g and 4 of group g + 2,
-    // the order the S^T layout leaves them in) are 16 consecutive bytes.
-    auto vpos = [](int key) { return (key & ~12) | ((key & 4) << 1) | ((key & 8) >> 1); };
-    auto lstore_v = [&](int buf) {
-        uint8_t *vt = lds + 2 * KSZ + buf * VSZ;
-#pragma unroll
-        for (int it = 0; it < VI; it++) {
-            const int idx = it * AT + tid, key = 2 * (idx % (AK / 2)), ch = idx / (AK / 2);
-            if (idx >= VN) continue;
-            const uint32_t av[4] = {va[it].x, va[it].y, va[it].z, va[it].w};
-            const uint32_t bv[4] = {vb[it].x, vb[it].y, vb[it].z, vb[it].w};
-#pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const uint32_t lo = (e & 1) ? av[e / 2] >> 16 : av[e / 2] & 0xFFFFu;
-                const uint32_t hi = (e & 1) ? bv[e / 2] >> 16 : bv[e / 2] & 0xFFFFu;
-                *(uint32_t *)(vt + (8 * ch + e) * VSTR + vpos(key) * 2) = lo | (hi << 16);
-            }
-        }
+    auto load_v = [&](int it, int slot, int e) {
+        const uint32_t off = (voff[it] + (uint32_t)tile_of(e) * (AK * D * ES)) | oob(e >= 0);
+        if constexpr (DT == LX2V_DTYPE_BF16)
+            dma16_at(vsrc, vdst + slot * L::VSZ + it * (AT * 16), off);
+        else
+            raw8(vsrc, off, vr[it]);
     };
-    // S^T = K Q^T for the 64 keys in K buffer kb: keys 32 j + (8 g + 4 hf + r),
-    // r = 0..3, in registers 4 g + r of st[j].
-    // (the two 32-key blocks' MFMA chains alternate, so that no MFMA waits
-    // for the one just before it)
-    auto scores = [&](int kbuf, f32x16 *st) {
-        const uint8_t *ks = lds + kbuf * KSZ;
-        st[0] = (f32x16){};
-        st[1] = (f32x16){};
+    auto store_k = [&](int it, int slot) {
+        if constexpr (DT != LX2V_DTYPE_BF16)
+            *(u32x4 *)(lds + L::K0 + slot * L::KSZ + (it * (AT / 64) + wv) * L::KBS + lane * 16) = bf8(kr[it]);
+    };
+    auto store_v = [&](int it, int slot) {
+        if constexpr (DT != LX2V_DTYPE_BF16)
+            *(u32x4 *)(lds + L::V0 + slot * L::VSZ + (it * AT + tid) * 16) = bf8(vr[it]);
+    };
+    auto load_mask = [&](int e) {
+        const uint32_t mo = (moff + (uint32_t)tile_of(e) * (AK / 8)) | oob(state_of(e) == 2);
 #pragma unroll
-        for (int s = 0; s < QS; s++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const bf16x8 kf = __builtin_bit_cast(bf16x8, *(const u32x4 *)(ks + (32 * j + l32) * KSTR + (2 * s + hf) * 16));
-                st[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[s], st[j], 0, 0, 0);
-            }
+        for (int kb = 0; kb < 2; kb++) mwn[kb] = buffer_load_x1(msrc, mo + 4 * kb);
+    };
+    auto kfrag = [&](const uint8_t *const *kf, int s, int j) {
+        return __builtin_bit_cast(bf16x8, *(const u32x4 *)(kf[s & 1] + j * (32 / L::KB) * L::KBS + (s >> 1) * 64));
+    };
+    // V^T of keys 16 u + 4 hf + 0..3 and 16 u + 8 + 4 hf + 0..3: the 8 keys this
+    // lane's P^T registers of step u hold (the order the S^T layout leaves them in).
+    auto vfrag = [&](int slot, int u, int b) {
+        typedef short s16x4 __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) s16x4 *lp;
+        const uint8_t *const p = vfr[b] + slot * L::VSZ + u * (16 * D * 2);
+        const s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)p), y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(p + 8 * D * 2));
+        return __builtin_bit_cast(bf16x8, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
     };
 
-    // Mask tile kt's scores in place: a full tile with every pair allowed is
+    // Mask a tile's scores in place: a full tile with every pair allowed is
     // left alone; otherwise keys past sk and, in mixed tiles, pairs whose
     // mask bit is clear become -inf.  mwk: the tile's two mask words.
-    auto apply_mask = [&](f32x16 *st, int kt, const uint32_t *mwk) {
-        const int state = tstate(kt), k0 = kt * AK;
+    auto apply_mask = [&](f32x16 *st, int e, const uint32_t *mwk) {
+        const int state = state_of(e), k0 = tile_of(e) * AK;
         if (state == 1 && k0 + AK <= sk) return;
 #pragma unroll
         for (int j = 0; j < 2; j++) {
@@ -310,137 +322,208 @@ __global__ __launch_bounds__(AT) void k_attn_mfma(const void *__restrict__ Q, co
         }
     };
 
-    // Software pipeline: while tile t's softmax and O^T += V^T P^T run, the
-    // scores of tile t + 1 are computed (its K is already in LDS) and the K of
-    // tile t + 2 and V of t + 1 are loaded.  The MFMAs of S(t + 1) and the
-    // softmax of t are independent, so the matrix cores and the vector ALUs
-    // of a SIMD work at once.  Explicit vmcnt(0) after each store: the mask
-    // words were loaded before V and are complete once V is, but the
-    // compiler cannot see that across the loop's back edge.
-    int kt = next_tile(klo);
-    int kn = kt < khi ? next_tile(kt + 1) : khi;
-    f32x16 sc[2];  // scores of tile kt (raw q.k)
-    uint32_t mw[2] = {0u, 0u};
-    if (kt < khi) {
-        gload_k(kt);
-        gload_v(kt);
-        lstore_k(0);
-        lstore_v(0);
-        mw[0] = mwn[0];
-        mw[1] = mwn[1];
-        gload_k(kn);
-        lstore_k(1);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __syncthreads();
-    if (kt < khi) {
-        scores(0, sc);
-        apply_mask(sc, kt, mw);
-    }
-    __syncthreads();  // K buffer 0 is rewritten at the end of the first iteration
-    int kbi = 1, vbi = 0;  // K buffer holding K(kn); V buffer holding V(kt)
+    // One key tile t per iteration:
+    //   O^T += V(t-1)^T P(t-1)^T   V(t-1) in V slot P ^ 1 (P = t & 1)
+    //   softmax of S(t)            in `cur`, P(t)^T into `pout`
+    //   S(t+1) = K(t+1) Q^T        K(t+1) in K slot ks, into `nxt`
+    // while V(t+1) is loaded into V slot P ^ 1 and K(t+3) into the K slot that
+    // held K(t).  The three are independent, and the code deals them out by hand: a step is one MFMA,
+    // the LDS read of the fragment that the MFMA RF - 1 steps on needs, and
+    // that step's share of the softmax, fenced so that the order stays.  The
+    // matrix cores and the vector ALU of a SIMD then both have work from each
+    // of its two waves at any time.
+    //
+    // One barrier per tile, at the first step of S(t+1): there every wave is past
+    // its reads of V(t-1) and K(t), and has V(t) and K(t+2) in LDS (loaded
+    // since the barrier before).  Between barriers a wave runs on from one
+    // tile into the next with RF - 1 fragments in flight, so no MFMA waits for
+    // LDS behind a barrier.
     const float tau = 8.0f;  // rescale O only when a query's max grows by more than 2^8
-    while (kt < khi) {
-        const int knn = kn < khi ? next_tile(kn + 1) : khi;
-        // loads for the stores at the end of this iteration (kOob when past the last tile)
+    constexpr int RF = 4;    // fragment registers (8 measured the same)
+    bf16x8 fr[RF];
+    uint32_t mw[2] = {0u, 0u};
+    int e0 = 0, e1 = 0, e2 = 0, e3 = 0, t = 0, ks = 0;
+    auto iter = [&](auto par, auto first, f32x16 *cur, f32x16 *nxt, const u32x4 *pin,
+                    u32x4 *pout) __attribute__((always_inline)) {
+        constexpr int P = decltype(par)::value;
+        constexpr int NPV = decltype(first)::value ? 0 : 4 * DB, NS = 2 * QS, NM = NPV + NS;
+        static_assert(NM % RF == 0 && NS > RF && 4 * DB >= RF, "the fragment ring runs on across tiles");
+        const uint8_t *const kf[2] = {kfr2[0] + ks * L::KSZ, kfr2[1] + ks * L::KSZ};
+        const int kold = ks == 0 ? 2 : ks - 1;  // K(t)'s slot
+        // fragment of step I of this tile; past its last step, V(t)'s
+        auto fetch = [&](auto i) {
+            constexpr int I = decltype(i)::value;
+            if constexpr (I < NPV)
+                fr[I % RF] = vfrag(P ^ 1, I / DB, I % DB);
+            else if constexpr (I < NM)
+                fr[I % RF] = kfrag(kf, (I - NPV) / 2, (I - NPV) % 2);
+            else
+                fr[I % RF] = vfrag(P, (I - NM) / DB, (I - NM) % DB);
+        };
+        constexpr int SBAR = NPV;  // the barrier's step
+        if constexpr (decltype(first)::value) static_for<RF - 1>(fetch);
+        const int e4 = entry(t + 4);
+        apply_mask(cur, e0, mw);
         __builtin_amdgcn_sched_barrier(0);
-        gload_k(knn);
-        gload_v(kn);
 
-        // S(kn), unconditionally (past the last tile it reads a stale buffer
-        // and is not used): a branch here would keep these MFMAs from being
-        // interleaved with the softmax below.
-        f32x16 sn[2];
-        scores(kbi, sn);
-        // The loads go between the first MFMAs of S(kn): issued back to back
-        // by all eight waves they held each wave's issue for hundreds of
-        // cycles at the top of every tile.
-        constexpr int NVM = (KI + 2 * VI) * (DT == LX2V_DTYPE_BF16 ? 1 : 2) + 2;
-#pragma unroll
-        for (int i = 0; i < NVM; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // an MFMA
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // a global load
-        }
-
-        // tile kt's scores were masked when they were computed
-        float tmax = -INFINITY;
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) tmax = fmaxf(tmax, sc[j][i]);
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64)) * c;
-        // The reference point moves only when the tile's max passes it by more
-        // than tau: p = 2^(s c - m) <= 2^tau in between, exact in f32, and O
-        // is rescaled far less often.  With no key allowed yet (m = -inf) any
-        // finite reference works: use 0.  The raw v_exp_f32 flushes results
-        // below 2^-126 to 0 (no contribution a softmax sum in f32 could
-        // register).
-        const float mn = tmax > m + tau ? tmax : m;
-        const float mref = mn == -INFINITY ? 0.0f : mn;
-        const float alpha = __builtin_amdgcn_exp2f(m - mref);
-        float psum = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[j][i], c, -mref));
-                sc[j][i] = p;
-                psum += p;
+        // Softmax of 32 scores: steps S0 .. SR - 1 take the max (from S0 on:
+        // the last MFMA of S(t) has then retired), SR the new reference
+        // point, the rest exponentials, sums and bf16 pairs.
+        constexpr int S0 = 1, SR = S0 + NM / 8, NB = NM - SR - 1;
+        auto x = [&](int v) -> float { return cur[v / 16][v % 16]; };
+        float tmax = -INFINITY, mn = m, mref = 0.0f, alpha = 1.0f, ps[2] = {0.0f, 0.0f};
+        float p[32];
+        // (the empty volatile asm statements keep a value's computation in
+        // its step: left alone, the compiler sinks it below the branch at the
+        // end of the iteration)
+        auto sum_pack = [&](int v) {
+            ps[v & 1] += p[v];
+            asm volatile("" : "+v"(ps[v & 1]));
+            if (v & 1) {
+                uint32_t w = pack_bf16x2(p[v - 1], p[v]);
+                asm volatile("" : "+v"(w));
+                pout[v / 8][(v % 8) / 2] = w;
             }
-        psum += __shfl_xor(psum, 32, 64);
-        lsum = lsum * alpha + psum;
+        };
+        static_for<NM>([&](auto ic) {
+            constexpr int I = decltype(ic)::value;
+            if constexpr (I < NPV) {
+                constexpr int u = I / DB, b = I % DB;
+                o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[I % RF], __builtin_bit_cast(bf16x8, pin[u]), o[b], 0, 0, 0);
+            } else {
+                constexpr int s = (I - NPV) / 2, j = (I - NPV) % 2;
+                if constexpr (s == 0) nxt[j] = (f32x16){};
+                nxt[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[I % RF], qf[s], nxt[j], 0, 0, 0);
+            }
+            if constexpr (I == SBAR) {
+                if constexpr (DT == LX2V_DTYPE_BF16)
+                    wait_vmcnt<0>();
+                else
+                    wait_vmcnt_lds0<0>();
+                asm volatile("s_barrier" ::: "memory");
+            }
+            fetch(std::integral_constant<int, I + RF - 1>{});
+            if constexpr (I == 0) load_mask(e1);
+            if constexpr (I > SBAR && I <= SBAR + KI) load_v(I - SBAR - 1, P ^ 1, e1);
+            if constexpr (I > SBAR + KI && I <= SBAR + 2 * KI) load_k(I - SBAR - KI - 1, kold, e3);
+            if constexpr (I >= S0 && I < SR) {
+#pragma unroll
+                for (int v = 32 * (I - S0) / (SR - S0); v < 32 * (I - S0 + 1) / (SR - S0); v += 2)
+                    tmax = fmaxf(fmaxf(tmax, x(v)), x(v + 1));
+            } else if constexpr (I == SR) {
+                // The reference point moves only when the tile's max passes it
+                // by more than tau: p = 2^(s c - m) <= 2^tau in between, exact
+                // in f32, and O is rescaled far less often.  With no key
+                // allowed yet (m = -inf) any finite reference works: use 0.
+                // The raw v_exp_f32 flushes results below 2^-126 to 0 (no
+                // contribution a softmax sum in f32 could register).
+                tmax = max_pair32(tmax) * c;
+                mn = tmax > m + tau ? tmax : m;
+                mref = mn == -INFINITY ? 0.0f : mn;
+                alpha = __builtin_amdgcn_exp2f(m - mref);
+            } else if constexpr (I > SR) {
+                constexpr int B = I - SR - 1, v0 = 32 * B / NB, v1 = 32 * (B + 1) / NB;
+#pragma unroll
+                for (int v = v0; v < v1; v++) {
+                    p[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(x(v), c, -mref));
+                    asm volatile("" : "+v"(p[v]));
+                    if (v > 0) sum_pack(v - 1);  // (one behind the exponential's latency)
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        sum_pack(31);
+#pragma unroll
+        for (int it = 0; it < KI; it++) {
+            store_v(it, P ^ 1);
+            store_k(it, kold);
+        }
+        lsum = lsum * alpha + (ps[0] + ps[1]);
         m = mn;
         if (__ballot(alpha != 1.0f)) {
+            asm volatile("" : "+v"(alpha));  // (the products stay behind the branch: hoisted, every tile pays for them)
 #pragma unroll
             for (int b = 0; b < DB; b++)
 #pragma unroll
                 for (int i = 0; i < 16; i++) o[b][i] *= alpha;
         }
-
-        // O^T += V^T P^T, four 16-key steps: step u = 2 j + t takes registers
-        // 8 t .. 8 t + 7 of sc[j], i.e. keys 32 j + 16 t + 4 hf + 0..3 and
-        // 32 j + 16 t + 8 + 4 hf + 0..3, which V^T holds as the 16 bytes at
-        // key position 16 u + 8 hf (vpos).  Step u + 1's V fragments are read
-        // while step u's MFMAs run.
-        const uint8_t *vt = lds + 2 * KSZ + vbi * VSZ;
-        auto vread = [&](int u, bf16x8 *vf) {
-#pragma unroll
-            for (int b = 0; b < DB; b++)
-                vf[b] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(vt + (32 * b + l32) * VSTR + (16 * u + 8 * hf) * 2));
-        };
-        bf16x8 vcur[DB], vnxt[DB];
-        vread(0, vcur);
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            if (u < 3) vread(u + 1, vnxt);
-            __builtin_amdgcn_sched_barrier(0);
-            const f32x16 &sp = sc[u >> 1];
-            const int t = u & 1;
-            const u32x4 pw = (u32x4){pack_bf16x2(sp[8 * t + 0], sp[8 * t + 1]), pack_bf16x2(sp[8 * t + 2], sp[8 * t + 3]),
-                                     pack_bf16x2(sp[8 * t + 4], sp[8 * t + 5]), pack_bf16x2(sp[8 * t + 6], sp[8 * t + 7])};
-            const bf16x8 pf = __builtin_bit_cast(bf16x8, pw);
-#pragma unroll
-            for (int b = 0; b < DB; b++) o[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vcur[b], pf, o[b], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            if (u < 3)
-#pragma unroll
-                for (int b = 0; b < DB; b++) vcur[b] = vnxt[b];
-        }
-        // K(kt) and V of the previous tile were last read before the previous
-        // barrier (stores past the last tile write zeros, unused)
-        lstore_k(kbi ^ 1);
-        lstore_v(vbi ^ 1);
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
         mw[0] = mwn[0];
         mw[1] = mwn[1];
-        if (kn < khi) apply_mask(sn, kn, mw);
-        __syncthreads();
-        sc[0] = sn[0];
-        sc[1] = sn[1];
-        kbi ^= 1;
-        vbi ^= 1;
-        kt = kn;
-        kn = knn;
+        e0 = e1;
+        e1 = e2;
+        e2 = e3;
+        e3 = __builtin_amdgcn_readfirstlane(e4);
+        t++;
+        ks = ks == 2 ? 0 : ks + 1;
+    };
+
+    if (n > 0) {
+        using std::integral_constant;
+        constexpr integral_constant<int, 0> c0{};
+        constexpr integral_constant<int, 1> c1{};
+        constexpr integral_constant<bool, true> first{};
+        constexpr integral_constant<bool, false> later{};
+        e0 = __builtin_amdgcn_readfirstlane(entry(0));
+        e1 = __builtin_amdgcn_readfirstlane(entry(1));
+        e2 = __builtin_amdgcn_readfirstlane(entry(2));
+        e3 = __builtin_amdgcn_readfirstlane(entry(3));
+        // Tiles 0 .. 2 of K into slots 0 .. 2, V of tile 0, S(0); tile t + 1's K
+        // is then in slot (t + 1) % 3 = ks.
+        f32x16 sa[2], sb[2];
+        u32x4 pa[4], pb[4];
+        auto begin = [&](int vslot, f32x16 *cur) __attribute__((always_inline)) {
+#pragma unroll
+            for (int it = 0; it < KI; it++) {
+                load_v(it, vslot, e0);
+                store_v(it, vslot);
+            }
+#pragma unroll
+            for (int tl = 0; tl < 3; tl++)
+#pragma unroll
+                for (int it = 0; it < KI; it++) {
+                    load_k(it, tl, tl == 0 ? e0 : (tl == 1 ? e1 : e2));
+                    store_k(it, tl);
+                }
+            load_mask(e0);
+            wait_vmcnt<0>();
+            mw[0] = mwn[0];
+            mw[1] = mwn[1];
+            __syncthreads();
+            cur[0] = cur[1] = (f32x16){};
+#pragma unroll
+            for (int s = 0; s < QS; s++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    cur[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfrag(kfr2, s, j), qf[s], cur[j], 0, 0, 0);
+            ks = 1;
+        };
+        // Tile 0 takes the V slot that lets the loop below, two tiles a turn,
+        // end on slot 0: slot 0 for odd n, slot 1 (and one more tile before
+        // the loop) for even n.
+        if (n & 1) {
+            begin(0, sa);
+            iter(c0, first, sa, sb, pb, pa);
+        } else {
+            begin(1, sb);
+            iter(c1, first, sb, sa, pa, pb);
+            iter(c0, later, sa, sb, pb, pa);
+        }
+        while (t < n) {
+            iter(c1, later, sb, sa, pa, pb);
+            iter(c0, later, sa, sb, pb, pa);
+        }
+        // the last tile's O^T += V^T P^T, from V slot 0 (its first fragments
+        // are in `fr`)
+        static_for<4 * DB>([&](auto ic) {
+            constexpr int I = decltype(ic)::value;
+            if constexpr (I + RF - 1 < 4 * DB) fr[(I + RF - 1) % RF] = vfrag(0, (I + RF - 1) / DB, (I + RF - 1) % DB);
+            o[I % DB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr[I % RF], __builtin_bit_cast(bf16x8, pa[I / DB]), o[I % DB], 0, 0, 0);
+        });
+    }
+    {  // the other half of each query's keys
+        uint32_t a = __float_as_uint(lsum), b = a;
+        swap32(a, b);
+        lsum = __uint_as_float(a) + __uint_as_float(b);
     }
 
     if (!qin) return;

@@ -77,6 +77,23 @@ def test_attention_mfma(be, heads, sq, sk, d, dtype):
     assert_close(got, _want(q, k, v), *MFMA_TOL, what=f"attention {heads}x{sq}x{sk}x{d}")
 
 
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("dtype", [H.DTYPE_F32, H.DTYPE_BF16])
+@pytest.mark.parametrize("sk", [1, 63, 64, 65, 128, 129, 192, 200, 256, 321])
+def test_attention_key_tile_counts(be, sk, dtype, d):
+    """One to six 64-key tiles, whole and ragged (the pipeline's first, even
+    and odd last tiles), one query past a 256-query tile; with a mask too: its
+    odd key tiles skipped for most queries, partly open for the others."""
+    heads, sq = 2, 257
+    q, k, v = _qkv(9000 + sk + d, heads, sq, sk, d)
+    assert_close(_run(be, q, k, v, dtype=dtype), _want(q, k, v), *MFMA_TOL, what=f"sk {sk}")
+    tile = np.arange(sk) // 64
+    mask = np.broadcast_to(tile % 2 == 0, (sq, sk)).copy()
+    mask[256] = (np.arange(sk) % 3 != 1) | (np.arange(sk) == sk - 1)
+    got = _run(be, q, k, v, mask, dtype=dtype)
+    assert_close(got, _want(q, k, v, mask), *MFMA_TOL, what=f"masked sk {sk}")
+
+
 # The MFMA path against the reference's own f32 attention on the unrounded
 # f32 inputs (cpu/src/lib.rs:171-203): the deviation the bf16 operands and
 # bf16 P add.  Measured on gfx950 (printed by this test): rel-L2 2.95e-3 ..
