@@ -189,10 +189,7 @@ __global__ __launch_bounds__(AT) void k_attn_mfma(const void *__restrict__ Q, co
         }
         if (lane == 0) nlist = total;
     }
-    // Q in registers before the loop: otherwise the first use of qf in every
-    // iteration waits for all loads in flight, the next tile's included.
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __syncthreads();
+    if (tlds) __syncthreads();
     const int nall = tlds ? nlist : nkt;
     // This workgroup's entries [i0, i0 + n): all, or in split mode those from
     // the floor(p n / S)-th to the floor((p + 1) n / S)-th (piece p).
@@ -485,6 +482,8 @@ __global__ __launch_bounds__(AT) void k_attn_mfma(const void *__restrict__ Q, co
                     store_k(it, tl);
                 }
             load_mask(e0);
+            // (Q too: its first use in every iteration would otherwise wait
+            // for all loads in flight, the next tile's included)
             wait_vmcnt<0>();
             mw[0] = mwn[0];
             mw[1] = mwn[1];
@@ -564,28 +563,43 @@ __global__ __launch_bounds__(AT) void k_attn_mfma(const void *__restrict__ Q, co
             amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
             const int k = mx_exponent(amax);
             const float msc = mx_scale(k);
+            // lane l ends with the block's codes 0..15, lane l + 32 with 16..31
+            uint32_t w[4];
 #pragma unroll
-            for (int g = 0; g < 4; g++)
-                *(uint32_t *)((uint8_t *)out + row0 + 32 * b + 8 * g + 4 * hf) = quant4_sc(v + 4 * g, msc);
+            for (int g = 0; g < 4; g++) w[g] = quant4_sc(v + 4 * g, msc);
+            swap32(w[0], w[2]);
+            swap32(w[1], w[3]);
+            *(u32x4 *)((uint8_t *)out + row0 + 32 * b + 16 * hf) = (u32x4){w[0], w[2], w[1], w[3]};
             if (hf == 0) omx[mx_sidx(q, (head * D + 32 * b) / 32, omx_rows)] = (uint8_t)(k + 127);
         }
         return;
     }
+    const size_t oi = ((size_t)q * heads + head) * D;
 #pragma unroll
-    for (int b = 0; b < DB; b++)
+    for (int b = 0; b < DB; b++) {
+        if constexpr (ODT == LX2V_DTYPE_BF16) {
+            // d 8 g + 4 hf .. + 3 in registers 4 g .. + 3: lanes l and l + 32
+            // trade halves, lane l storing 8 d of an even g, lane l + 32 of
+            // the odd one beside it (32 contiguous bytes of the row)
 #pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const int d0 = 32 * b + 8 * g + 4 * hf;
-            const size_t oi = ((size_t)q * heads + head) * D + d0;
-            const float v0 = o[b][4 * g] * inv, v1 = o[b][4 * g + 1] * inv, v2 = o[b][4 * g + 2] * inv,
-                        v3 = o[b][4 * g + 3] * inv;
-            if constexpr (ODT == LX2V_DTYPE_BF16) {
-                typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-                *(u32x2_t *)((uint16_t *)out + oi) = (u32x2_t){pack_bf16x2(v0, v1), pack_bf16x2(v2, v3)};
-            } else {
-                *(f32x4 *)((float *)out + oi) = (f32x4){v0, v1, v2, v3};
+            for (int g = 0; g < 4; g += 2) {
+                uint32_t w[4];
+#pragma unroll
+                for (int h = 0; h < 4; h++) {
+                    const int r = 4 * (g + h / 2) + 2 * (h % 2);
+                    w[h] = pack_bf16x2(o[b][r] * inv, o[b][r + 1] * inv);
+                }
+                swap32(w[0], w[2]);
+                swap32(w[1], w[3]);
+                *(u32x4 *)((uint16_t *)out + oi + 32 * b + 8 * (g + hf)) = (u32x4){w[0], w[1], w[2], w[3]};
             }
+        } else {
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                *(f32x4 *)((float *)out + oi + 32 * b + 8 * g + 4 * hf) =
+                    (f32x4){o[b][4 * g] * inv, o[b][4 * g + 1] * inv, o[b][4 * g + 2] * inv, o[b][4 * g + 3] * inv};
         }
+    }
 }
 
 // Split mode's second pass: the S pieces of each (query, head) row
