@@ -1355,11 +1355,10 @@ __global__ __launch_bounds__(512, 1) void k_gemm_fp8_ov(const uint8_t *__restric
 //
 // vmcnt accounting: every stage issues LPS = 9 loads and every epilogue
 // ST stores (stores past M or N go to an out-of-range offset, so the count
-// is the same for every lane and tile; a dummy epilogue of ST out-of-range
-// stores follows the prologue loads for the first tile).  At the top of
-// stage g the loads of g + 1 and g + 2 may still be in flight, and, for the
-// first three stages of a tile, the previous tile's stores issued after
-// stage g's loads: the waits allow exactly those.
+// is the same for every lane and tile).  At the top of stage g the loads of
+// g + 1 and g + 2 may still be in flight, and, for the first three stages of
+// every tile but the workgroup's first, the previous tile's stores issued
+// after stage g's loads: the waits allow exactly those.
 //
 // Constraints (host): K % 64 == 0, K / 64 >= 4, N % 256 == 0, M N sizeof(TY)
 // < 2^31; bf16 or MX e4m3 output; per-token activations, per-channel weight
@@ -1589,16 +1588,13 @@ __global__ __launch_bounds__(256, 1) void k_gemm_fp8_w4(const uint8_t *__restric
         });
     };
 
-    // Prologue: the first NS - 1 stages, then the dummy epilogue's stores.
+    // Prologue: the first NS - 1 stages.
 #pragma unroll
     for (int st = 0; st < NS - 1; st++) {
 #pragma unroll
         for (int n = 0; n < LPS; n++) load(n, st);
         advance_issue();
     }
-#pragma unroll
-    for (int q = 0; q < ST; q++) buffer_store_b8(0, ry, kOob);
-
     int g = 0;  // global stage index of this workgroup's walk
     // One stage of the K loop.  The loop is skewed by one 64-byte slice:
     // after barrier g a wave contracts the slice before stage g's first
@@ -1606,9 +1602,9 @@ __global__ __launch_bounds__(256, 1) void k_gemm_fp8_w4(const uint8_t *__restric
     // each next slice while reading the one after it.  64-byte stages use
     // the two fragment sets by stage parity P (KT is even), 128-byte stages
     // by slice.
-    auto iter = [&](auto P, int kt) {
+    auto iter = [&](auto P, int kt, bool later) {  // later: not this workgroup's first tile
         constexpr int p = decltype(P)::value;
-        if (kt < NS - 1)
+        if (kt < NS - 1 && later)
             wait_vmcnt_lds0<(NS - 2) * LPS + ST>();
         else
             wait_vmcnt_lds0<(NS - 2) * LPS>();
@@ -1651,11 +1647,11 @@ __global__ __launch_bounds__(256, 1) void k_gemm_fp8_w4(const uint8_t *__restric
         tile_of(t, &m0, &n0);
         if constexpr (KK == 1) {
             for (int kt = 0; kt < KT; kt += 2) {
-                iter(std::integral_constant<int, 0>{}, kt);
-                iter(std::integral_constant<int, 1>{}, kt + 1);
+                iter(std::integral_constant<int, 0>{}, kt, t > 0);
+                iter(std::integral_constant<int, 1>{}, kt + 1, t > 0);
             }
         } else {
-            for (int kt = 0; kt < KT; kt++) iter(I0{}, kt);
+            for (int kt = 0; kt < KT; kt++) iter(I0{}, kt, t > 0);
         }
         // the tile's last slice (set 1), from registers, then its epilogue
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): its fragments
