@@ -2123,10 +2123,10 @@ void launch_dma_idx(int idx, hipStream_t s, const uint8_t *a, const float *sa, c
             // read and a write besides (kv2 12.4 -> 9.7 us, 880 x 14336 ->
             // 3072 76 -> 51 us); per-channel, four waves are as fast or faster
             if (mx.wgs)
-                launch_dma<128, 128, 4, 2, 128, 3, 1, false, false, true>(s, a, sa, b, sb, bias, act, y, y_dtype, M, N,
+                launch_dma<128, 128, 4, 2, 128, 3, 1, false, true, true>(s, a, sa, b, sb, bias, act, y, y_dtype, M, N,
                                                                           K, mx);
             else
-                launch_dma<128, 128, 2, 2, 128, 3, 1>(s, a, sa, b, sb, bias, act, y, y_dtype, M, N, K, mx);
+                launch_dma<128, 128, 2, 2, 128, 3, 1, true, true>(s, a, sa, b, sb, bias, act, y, y_dtype, M, N, K, mx);
             break;
         default: break;  // 6 .. 9: launch_pt / launch_ov / launch_w4 (need the CU count)
     }
@@ -2241,16 +2241,22 @@ double cfg_cost(const CfgCost &c, size_t tiles, size_t num_cu, size_t K) {
     return t;
 }
 
-// The configurations with MX-activation / MX-output kernels.  The 128 x 256
+// The configurations with MX-activation / MX-output kernels.  The 128 x 128
+// one-per-CU tile (10) takes both: it is the choice wherever the larger
+// tiles leave CUs idle (MX input, 256 x 128 or 128 x 256 tile -> 128 x 128:
+// 880 x 14336 -> 3072 70.5 -> 48.0 us, 1560 x 8960 -> 1536 45.8 -> 30.5, 1560
+// x 1536 -> 1536 12.2 -> 8.7; MX output, 300 x 3072 -> 3072 13.4 -> 12.5,
+// there against the three-per-CU tile).  The 128 x 256
 // two-per-CU tile takes no MX activations: their scale handling needs more
 // than the 128 VGPRs two workgroups per CU leave a wave (its one-per-CU
 // version, 1, has 256).
-bool mx_capable(int idx, bool mx_in) { return idx <= 1 || idx == 3 || ((idx == 4 || idx == 6) && !mx_in); }
+bool mx_capable(int idx, bool mx_in) { return idx <= 1 || idx == 3 || idx == 10 || ((idx == 4 || idx == 6) && !mx_in); }
 // The configurations built with grouped weight scales (128-byte stages, one
-// workgroup per CU: the partial sums need the registers); MX output on the
-// 256 x 128 and 128 x 256 tiles, MX activations on the one-shot ones.
+// workgroup per CU: the partial sums need the registers); MX output of
+// per-token activations on the 256 x 128 and 128 x 256 tiles, MX activations
+// on the one-shot ones.
 bool grouped_capable(int idx, bool mx, bool mx_in) {
-    return mx_in ? idx <= 1 : (idx <= 1 || idx == 6 || (idx == 10 && !mx));
+    return mx_in ? idx <= 1 || idx == 10 : (idx <= 1 || idx == 6 || (idx == 10 && !mx));
 }
 // The overlapped-epilogue kernel (k_gemm_fp8_ov): per-token activations,
 // per-channel or group-128 weight scales, bf16 or MX e4m3 output, whole 128-channel
@@ -2297,7 +2303,7 @@ Fp8Plan plan_gemm_fp8(int num_cu, size_t M, size_t N, size_t K, bool mx, bool mx
         // CUs without a reduction) is cheaper by the model below; a forced
         // split count always splits
         bool split = S >= 2 && (size_t)M * N * S * 4 < (1ull << 31);
-        if (split && mode < 2 && y_dtype != LX2V_DTYPE_MXE4M3) {  // (no MX output on that tile)
+        if (split && mode < 2) {
             const size_t t10 = ((M + 127) / 128) * (N / 128);
             const double c10 = cfg_cost(kAuto[sizeof(kAuto) / sizeof(kAuto[0]) - 1], t10, (size_t)num_cu, K);
             // the split's tiles (one round) plus the partials' store and reduction

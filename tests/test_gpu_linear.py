@@ -327,6 +327,34 @@ def test_fp8_mx_input_forced_vs_config0(be, monkeypatch, group, act, ydt):
                      what=f"c1 MX input (group {g}) vs oracle")
 
 
+@pytest.mark.parametrize("group,x_mx,ydt", [("channel", True, H.DTYPE_BF16), ("channel", True, H.DTYPE_MXE4M3),
+                                            ("channel", False, H.DTYPE_MXE4M3), (128, True, H.DTYPE_F32),
+                                            (128, True, H.DTYPE_MXE4M3)])
+@pytest.mark.parametrize("M,N", [(1, 32), (128, 128), (129, 160), (385, 1056)])
+def test_fp8_mx_128x128_vs_config0(be, monkeypatch, M, N, group, x_mx, ydt):
+    """The 128 x 128 one-per-CU tile (configuration 10) with MX input and / or
+    output against the 256 x 128 tile (0), bit for bit: one row, whole tiles,
+    one row past a tile, ragged columns."""
+    K = 512
+    g = K if group == "channel" else 128
+    _, q, s = fp8_weight(3242 + N, N, K, g)
+    w, bb = be.weight_fp8(q, s, N, K, g), be.upload(normal(3243, N, 0.01))
+    xb = be.upload(normal(3241 + M, M * K).reshape(M, K))
+    xq = xb
+    if x_mx:
+        xq = be.alloc_mx(M, K)
+        be.quantize_mx(xb, 0, M, xq)
+
+    def run(c):
+        monkeypatch.setenv("LIGHTX2V_HIP_FP8_CFG", str(c))
+        y = be.alloc_mx(M, N) if ydt == H.DTYPE_MXE4M3 else be.alloc(M * N, ydt)
+        _, names = _kernels(be, lambda: be.linear(xq, 0, M, w, bb, H.ACT_GELU_TANH, y, 0))
+        assert any(f".c{c}" in k for k in names), names
+        return be.download_mx(y, M, N) if ydt == H.DTYPE_MXE4M3 else (u32(be.download(y)),)
+
+    assert all(np.array_equal(a, b) for a, b in zip(run(0), run(10)))
+
+
 def test_fp8_no_bias(be):
     M, K, N = 96, 640, 320
     x = normal(8, M * K).reshape(M, K)
