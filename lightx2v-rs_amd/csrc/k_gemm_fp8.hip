@@ -2282,7 +2282,10 @@ bool w4_capable(size_t M, size_t N, size_t K, bool mx_in, bool grouped, int y_dt
 Fp8Plan plan_gemm_fp8(int num_cu, size_t M, size_t N, size_t K, bool mx, bool mx_in, bool grouped, int y_dtype,
                       int act, bool residual, bool allow_split) {
     Fp8Plan p;
-    if (K % 128 != 0) return p;  // the register-staged kernel
+    if (K % 128 != 0) {  // the register-staged kernel
+        p.cost_us = (double)K / 64 * 0.45 + 6.0;
+        return p;
+    }
     // Split K where even the 256 x 128 tiles leave at least half the CUs
     // idle and K is long: S workgroups per tile (S <= CUs / tiles, >= 32
     // stages each, <= 8), their partial sums reduced by a second pass.  The
@@ -2303,6 +2306,7 @@ Fp8Plan plan_gemm_fp8(int num_cu, size_t M, size_t N, size_t K, bool mx, bool mx
         // CUs without a reduction) is cheaper by the model below; a forced
         // split count always splits
         bool split = S >= 2 && (size_t)M * N * S * 4 < (1ull << 31);
+        double split_us = 0.0;  // a forced split: no model, as a pinned configuration
         if (split && mode < 2) {
             const size_t t10 = ((M + 127) / 128) * (N / 128);
             const double c10 = cfg_cost(kAuto[sizeof(kAuto) / sizeof(kAuto[0]) - 1], t10, (size_t)num_cu, K);
@@ -2310,10 +2314,12 @@ Fp8Plan plan_gemm_fp8(int num_cu, size_t M, size_t N, size_t K, bool mx, bool mx
             const double busy = (double)std::min<size_t>(tiles * S, (size_t)num_cu) / num_cu;
             const double cs = (double)(kts / S) * (0.40 + 0.38 * busy) + 5.3 + 10.0;
             split = cs <= c10;
+            split_us = cs;
         }
         if (split) {
             p.kernel = 0;
             p.splits = (int)S;
+            p.cost_us = split_us;
             return p;
         }
     }
@@ -2332,7 +2338,7 @@ Fp8Plan plan_gemm_fp8(int num_cu, size_t M, size_t N, size_t K, bool mx, bool mx
     double best = 0.0;
     auto take = [&](int idx, double t) {
         if (p.kernel < 0 || t < best * 0.9999) {  // ties keep the earlier
-            best = t;
+            best = p.cost_us = t;
             p.kernel = idx;
         }
     };

@@ -14,9 +14,11 @@
 // operand roles (weights = MFMA A operand, so the epilogue writes four
 // consecutive channels per lane) follow k_gemm_fp8.hip, with a 64-element K
 // stage (128 bytes of bf16 per row).
+#include <algorithm>
 #include <utility>
 
 #include "gemm_common.hpp"
+#include "w16_dequant.hpp"
 
 // Cache-policy bits of the LDS-staged epilogue's stores (buffer_store: 1 =
 // sc0, 2 = nt, 16 = sc1; the values written are the same for every policy):
@@ -346,79 +348,7 @@ void launch_tile(hipStream_t s, const void *x, int x_dtype, const lx2v_hip_weigh
 //   slot kt - 1 used; MFMAs.
 
 constexpr int BKE = 64;        // K elements per stage
-// Q4 with every zero 8 (lx2v_hip_weight::zero8): the same codes and scales,
-// no zeros loaded (a format id of this file only)
-constexpr int kWfmtQ4Sym = 100;
 constexpr int XRB = BKE * 2;   // bytes per LDS tile row (bf16)
-
-// 16 consecutive K elements of one weight row, as 8 packed bf16 pairs
-// (element 2i low), each rounded from the reference's f32 dequantization
-// (quant.rs:183-191, 279-289, 432-440): c = 16 code bytes (Q8, FP8) or 8
-// (Q4, in c.x, c.y), s / z = the group's scale / zero.
-template <int WF>
-__device__ __forceinline__ void unit_dequant(u32x4 c, float s, float z, uint32_t (&o)[8]) {
-    const uint32_t w[4] = {c.x, c.y, c.z, c.w};
-    if constexpr (WF == LX2V_WFMT_Q8) {
-        // byte ^ 0x80 reads as q + 128 unsigned, and fma(q + 128, s, -128 s)
-        // rounds the exact q * s once (128 s is exact): the reference's q * s.
-        const float nb = -128.0f * s;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const uint32_t b = w[q] ^ 0x80808080u;
-            const float f0 = __builtin_fmaf((float)(b & 0xFFu), s, nb);
-            const float f1 = __builtin_fmaf((float)((b >> 8) & 0xFFu), s, nb);
-            const float f2 = __builtin_fmaf((float)((b >> 16) & 0xFFu), s, nb);
-            const float f3 = __builtin_fmaf((float)(b >> 24), s, nb);
-            o[2 * q] = pack_bf16x2(f0, f1);
-            o[2 * q + 1] = pack_bf16x2(f2, f3);
-        }
-    } else if constexpr (WF == kWfmtQ4Sym) {
-        // zero 8: (c - 8) s is exact before its one rounding, and so is
-        // fma(c, s, -8 s) (8 s is exact): the same f32 value
-        const float nb = -8.0f * s;
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const uint32_t lo = w[q] & 0x0F0F0F0Fu, hi = (w[q] >> 4) & 0x0F0F0F0Fu;
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const float e0 = __builtin_fmaf((float)((lo >> (8 * b)) & 0xFFu), s, nb);
-                const float e1 = __builtin_fmaf((float)((hi >> (8 * b)) & 0xFFu), s, nb);
-                o[4 * q + b] = pack_bf16x2(e0, e1);
-            }
-        }
-        (void)z;
-    } else if constexpr (WF == LX2V_WFMT_Q4) {
-        // element 2i in the low nibble of byte i (quant.rs:305-311)
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const uint32_t lo = w[q] & 0x0F0F0F0Fu, hi = (w[q] >> 4) & 0x0F0F0F0Fu;
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const float e0 = ((float)((lo >> (8 * b)) & 0xFFu) - z) * s;
-                const float e1 = ((float)((hi >> (8 * b)) & 0xFFu) - z) * s;
-                o[4 * q + b] = pack_bf16x2(e0, e1);
-            }
-        }
-    } else {
-        // e4m3 through the hardware OCP decode; the reference decodes
-        // exponent field 0 as m * 2^-12, an eighth of OCP's m * 2^-9.
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            typedef float f32x2_t __attribute__((ext_vector_type(2)));
-            const f32x2_t a = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[q], false);
-            const f32x2_t b = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[q], true);
-            float f[4] = {a.x, a.y, b.x, b.y};
-            const uint32_t e = w[q] & 0x78787878u;
-            if ((e - 0x01010101u) & ~e & 0x80808080u) {  // some byte has exponent field 0
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-                    if (((e >> (8 * k)) & 0xFFu) == 0) f[k] *= 0.125f;
-            }
-            o[2 * q] = pack_bf16x2(f[0] * s, f[1] * s);
-            o[2 * q + 1] = pack_bf16x2(f[2] * s, f[3] * s);
-        }
-    }
-}
 
 template <int BM, int BN, int WGM, int WGN, int NS, int WF, typename TY, int KE>
 __global__ __launch_bounds__(64 * WGM * WGN, 1) void k_gemm_w16_dma(const uint16_t *__restrict__ X,
@@ -979,6 +909,14 @@ int plan_gemm_w16_dma(int num_cu, size_t M, size_t N) {
     return pick;
 }
 
+// 256 x 128 and 128 x 256 tiles cost about 0.88 us per 64-element stage, the
+// 256 x 256 one 1.55 (M 128 .. 1560, K 512 .. 14336: within 15%).
+double gemm_w16_dma_cost_us(int num_cu, size_t M, size_t N, size_t K) {
+    const DmaCfg &c = kDmaW16[plan_gemm_w16_dma(num_cu, M, N)];
+    const size_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    return (double)((tiles + num_cu - 1) / num_cu) * ((double)K / 64 * (c.bm * c.bn > 256 * 128 ? 1.55 : 0.88) + 4.0);
+}
+
 void launch_gemm_w16_dma(hipStream_t s, int cfg, const uint16_t *x, const lx2v_hip_weight *w, const float *bias,
                          int act, void *y, int y_dtype, size_t M) {
     launch_dma_idx(cfg, s, x, w, bias, act, y, y_dtype, (int)M);
@@ -987,6 +925,13 @@ void launch_gemm_w16_dma(hipStream_t s, int cfg, const uint16_t *x, const lx2v_h
 bool gemm_bf16_supported(size_t M, size_t N, size_t K) {
     return M > 0 && N > 0 && K >= BKE && K % BKE == 0 && M * K * 2 < (1ull << 31) && N * K * 2 < (1ull << 31) &&
            M < (1u << 30) && N < (1u << 30);
+}
+
+// One round of 128 x 128 tiles: 0.41 us per 64-element stage and 3.5 us (512 x
+// 4096 -> 1536 29.8 us, 512 x 1536 -> 1536 13.3).
+double gemm_bf16_cost_us(int num_cu, size_t M, size_t N, size_t K) {
+    const size_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+    return (double)((tiles + num_cu - 1) / num_cu) * ((double)K / 64 * 0.41 + 3.5);
 }
 
 // 256 x 128 (8 waves), 128 x 256 (8 waves) or 128 x 128 (4 waves): the one

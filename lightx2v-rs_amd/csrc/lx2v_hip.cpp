@@ -1921,6 +1921,18 @@ static int act_quant_into_ws(lx2v_hip_ctx *ctx, const void *x, int dtype, size_t
 // scr: the no-alloc variant -- every workspace comes from this device
 // memory (bias staging first, then the activations' e4m3 codes and row
 // scales or their bf16 copy), and the call fails cleanly if it is too small.
+// Whether the few-rows kernel takes an FP8 linear, decided against the plan
+// linear itself would make (linear_residual asks the same question, so that
+// both sum in the same order).
+static bool few_rows_fp8(const lx2v_hip_ctx *ctx, size_t rows, const lx2v_hip_weight *w, bool x_mx, bool y_mx, bool grouped,
+                         int y_dtype, int act) {
+    const size_t N = w->rows, K = w->cols;
+    const Fp8Plan p = plan_gemm_fp8(ctx->num_cu, rows, N, K, x_mx || y_mx, x_mx, grouped, y_dtype, act, false, true);
+    if (p.splits > 1 && p.cost_us == 0.0) return false;  // a forced split
+    // (group-128 and MX stages of the few-tile configurations run slower than modelled)
+    return gemm_rows_chosen(RowsKind::Fp8, ctx->num_cu, rows, N, K, p.cost_us * (grouped ? 1.4 : x_mx ? 1.2 : 1.0));
+}
+
 static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, size_t rows, const lx2v_hip_weight *w,
                       const lx2v_hip_buf *bias, int act, lx2v_hip_buf *y, size_t y_row, const float *gate,
                       const lx2v::Scratch *scr = nullptr) {
@@ -1986,6 +1998,16 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
             plan.kernel != 10)  // built with grouped scales
             return fail(LX2V_ERR_UNSUPPORTED, "no grouped-scale fp8 kernel for configuration %d", plan.kernel);
     }
+    // Few rows: the kernels that read the weight once, on the same operands.
+    bool few = false;
+    if (e4m3_path)
+        few = fp8_mfma && few_rows_fp8(ctx, rows, w, x_mx, y_mx, fp8_grouped, y->dtype, act);
+    else if (native_bf16 || gemm_w16_dma_supported(w, rows))
+        few = gemm_rows_chosen(x->dtype == LX2V_DTYPE_F32 ? RowsKind::F32Act : native_bf16 ? RowsKind::Native : RowsKind::W16,
+                               ctx->num_cu, rows, N, K,
+                               (native_bf16 ? gemm_bf16_cost_us(ctx->num_cu, rows, N, K) : gemm_w16_dma_cost_us(ctx->num_cu, rows, N, K)) +
+                                   (x->dtype == LX2V_DTYPE_F32 ? 2.5 : 0.0));  // the tiles' pass that rounds f32 rows to bf16
+    if (few) plan.splits = 1;
     // Workspaces, each piece 256-byte aligned: a bf16 bias's f32 copy; the
     // activations' e4m3 codes and row scales, or their bf16 copy; split K's
     // f32 partial sums.  The no-alloc variant lays them out in that order in
@@ -1994,7 +2016,7 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t s_bias = bias && bias->dtype != LX2V_DTYPE_F32 ? al(N * 4) : 0;
     const size_t s_act = e4m3_path ? (x->quantized() ? 0 : al(rows * K) + al(rows * 4))
-                                   : ((gemm_w16_dma_supported(w, rows) || native_bf16) && x->dtype == LX2V_DTYPE_F32
+                                   : (!few && (gemm_w16_dma_supported(w, rows) || native_bf16) && x->dtype == LX2V_DTYPE_F32
                                           ? al(rows * K * 2)
                                           : 0);
     const size_t s_part = plan.splits > 1 ? al((size_t)plan.splits * rows * N * 4) : 0;
@@ -2070,9 +2092,13 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
             // e.g. "gemm_fp8_e4m3.c0.g128.mxout".
             char pname[64];
             char cfg[8] = "creg";  // the register-staged kernel (K % 128 != 0)
-            if (plan.kernel >= 0) snprintf(cfg, sizeof cfg, plan.splits > 1 ? "c%dk%d" : "c%d", plan.kernel, plan.splits);
+            if (few)
+                snprintf(cfg, sizeof cfg, "rows");
+            else if (plan.kernel >= 0) snprintf(cfg, sizeof cfg, plan.splits > 1 ? "c%dk%d" : "c%d", plan.kernel, plan.splits);
             snprintf(pname, sizeof pname, "gemm_fp8_e4m3.%s%s%s%s%s", cfg, fp8_grouped ? ".g128" : "", x_mx ? ".mxin" : "", y_mx ? ".mxout" : "", gate ? ".res" : "");
             if (int rc = run(ctx, pname, [&] {
+                    if (few)
+                        return launch_gemm_rows_fp8(ctx->stream, q, s, w, fp8_grouped, bp, act, yp, y->dtype, rows, mx);
                     launch_gemm_fp8(ctx->stream, ctx->num_cu, plan, q, s, (const uint8_t *)w->codes,
                                     fp8_grouped ? w->glast : w->scales, bp, act, yp, y->dtype, rows, N, K, mx);
                 }))
@@ -2086,6 +2112,11 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
                 return rc;
         }
         return ok();
+    }
+    if (few) {
+        const char *name = w->fmt == LX2V_WFMT_Q8 ? "gemm_w16_q8.rows" : w->fmt == LX2V_WFMT_Q4 ? "gemm_w16_q4.rows"
+                           : w->fmt == LX2V_WFMT_FP8 ? "gemm_w16_fp8.rows" : "gemm_bf16_native.rows";
+        return run(ctx, name, [&] { launch_gemm_rows_w16(ctx->stream, xp, x->dtype, w, bp, act, yp, y->dtype, rows); });
     }
     // bf16 activations for the direct-to-LDS kernels: f32 ones rounded (RNE,
     // as the register-staged loader would) into the workspace.
@@ -2193,13 +2224,14 @@ int lx2v_hip_linear_noalloc(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_r
 // linear itself would not split K (its sums would then be added in another
 // order than the fused kernel's; the pair keeps the two equal).
 static bool linear_fusable(const lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t rows, const lx2v_hip_weight *w,
-                           const lx2v_hip_buf *h) {
+                           const lx2v_hip_buf *h, int act) {
     const size_t N = w->rows, K = w->cols;
     const bool x_mx = x->dtype == LX2V_DTYPE_MXE4M3;
     const bool grouped = w->group != K;
     if (w->fmt != LX2V_WFMT_FP8 || h->quantized() || !gemm_fp8_supported(rows, N, K)) return false;
     if (grouped && !(w->gratio_ok && gemm_fp8_grouped_supported(rows, N, K, w->group))) return false;
     if (!(ctx->fp8_act == LX2V_FP8_ACT_E4M3 || x->quantized())) return false;
+    if (few_rows_fp8(ctx, rows, w, x_mx, false, grouped, h->dtype, act)) return true;  // that kernel has the add
     if (plan_gemm_fp8(ctx->num_cu, rows, N, K, x_mx, x_mx, grouped, h->dtype, LX2V_ACT_NONE, false, true).splits > 1)
         return false;
     return gemm_fp8_residual_ok(plan_gemm_fp8(ctx->num_cu, rows, N, K, x_mx, x_mx, grouped, h->dtype, LX2V_ACT_NONE, true));
@@ -2223,7 +2255,7 @@ int lx2v_hip_linear_residual(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_
     if (int rc = set_dev(ctx)) return rc;
     const float *g = nullptr;  // slot 2 of the staging: linear's bias conversion uses slot 0
     if (int rc = param_f32(ctx, mods, gate * N, N, 2, &g, "mods (gate)")) return rc;
-    if (linear_fusable(ctx, x, rows, w, h)) return linear_run(ctx, x, x_row, rows, w, bias, act, h, h_row, g);
+    if (linear_fusable(ctx, x, rows, w, h, act)) return linear_run(ctx, x, x_row, rows, w, bias, act, h, h_row, g);
     // Elsewhere: the linear into a workspace of h's dtype, then the add.
     auto &st = ctx->resid;
     if (int rc = ensure(ctx, &st.ptr, &st.bytes, rows * N * h->elem_bytes(), "residual workspace alloc")) return rc;

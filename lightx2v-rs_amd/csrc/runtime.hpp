@@ -295,6 +295,7 @@ struct Fp8Plan {
     // their f32 partial sums in Fp8Mx::part, summed by a second pass that
     // applies the scales, bias, activation and output form
     int splits = 1;
+    double cost_us = 0.0;  // modelled time (0: a pinned configuration)
 };
 // MX e4m3 operands of a launch: A's block scales ([K / 128][a_rows][4],
 // a_len bytes readable from a; a_scale is then null) and/or the output's
@@ -332,6 +333,19 @@ void launch_gemm_fp8(hipStream_t s, int num_cu, const Fp8Plan &p, const uint8_t 
                      const uint8_t *b, const float *b_scale, const float *bias, int act, void *y,
                      int y_dtype, size_t M, size_t N, size_t K, const Fp8Mx &mx);
 
+// k_gemm_rows.hip: linear over few rows, every weight format (K % 64 == 0).
+// The fp8 one takes e4m3 / MX activations and per-channel or group-128
+// weights (`grouped`: lx2v_hip_weight::sscale); the w16 one bf16 or f32
+// activations and the weights of launch_gemm_w16_dma, or a native weight's
+// bf16 copy.  gemm_rows_chosen: whether it takes a call that would otherwise
+// cost tile_us on the tile kernels.
+enum class RowsKind { Fp8, W16, Native, F32Act };  // F32Act: f32 activations of the bf16 MFMA kinds
+bool gemm_rows_chosen(RowsKind kind, int num_cu, size_t M, size_t N, size_t K, double tile_us);
+void launch_gemm_rows_fp8(hipStream_t s, const uint8_t *x, const float *x_scale, const lx2v_hip_weight *w, bool grouped,
+                          const float *bias, int act, void *y, int y_dtype, size_t M, const Fp8Mx &mx);
+void launch_gemm_rows_w16(hipStream_t s, const void *x, int x_dtype, const lx2v_hip_weight *w, const float *bias, int act,
+                          void *y, int y_dtype, size_t M);
+
 // k_gemm_w16.hip: bf16 MFMA with the weight dequantized to bf16 inside
 // the GEMM (Q8, Q4, FP8 with any group).  The direct-to-LDS kernel takes
 // bf16 activations with K % 64 == 0 and a group that is a multiple of 16;
@@ -343,11 +357,13 @@ void launch_gemm_w16(hipStream_t s, int num_cu, const void *x, int x_dtype,
                      size_t M);
 bool gemm_w16_dma_supported(const lx2v_hip_weight *w, size_t M);
 int plan_gemm_w16_dma(int num_cu, size_t M, size_t N);
+double gemm_w16_dma_cost_us(int num_cu, size_t M, size_t N, size_t K);  // modelled time of its choice
 void launch_gemm_w16_dma(hipStream_t s, int cfg, const uint16_t *x, const lx2v_hip_weight *w, const float *bias,
                          int act, void *y, int y_dtype, size_t M);
 // bf16 x bf16 (native f32 weights through their bf16 copy): X [M, K] and
 // W [N, K] bf16, K % 64 == 0.
 bool gemm_bf16_supported(size_t M, size_t N, size_t K);
+double gemm_bf16_cost_us(int num_cu, size_t M, size_t N, size_t K);  // modelled time of launch_gemm_bf16's choice
 void launch_gemm_bf16(hipStream_t s, int num_cu, const uint16_t *x, const uint16_t *w, const float *bias, int act,
                       void *y, int y_dtype, size_t M, size_t N, size_t K);
 
