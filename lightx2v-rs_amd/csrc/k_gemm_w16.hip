@@ -927,38 +927,61 @@ bool gemm_bf16_supported(size_t M, size_t N, size_t K) {
            M < (1u << 30) && N < (1u << 30);
 }
 
-// One round of 128 x 128 tiles: 0.41 us per 64-element stage and 3.5 us (512 x
-// 4096 -> 1536 29.8 us, 512 x 1536 -> 1536 13.3).
-double gemm_bf16_cost_us(int num_cu, size_t M, size_t N, size_t K) {
-    const size_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
-    return (double)((tiles + num_cu - 1) / num_cu) * ((double)K / 64 * 0.41 + 3.5);
-}
+namespace {
 
-// 256 x 128 (8 waves), 128 x 256 (8 waves) or 128 x 128 (4 waves): the one
-// that leaves the fewest idle tile slots over the rounds the grid takes, the
-// larger tile on ties.
-void launch_gemm_bf16(hipStream_t s, int num_cu, const uint16_t *x, const uint16_t *w, const float *bias, int act,
-                      void *y, int y_dtype, size_t M, size_t N, size_t K) {
-    struct Cfg {
-        int bm, bn;
-    };
-    const Cfg cfgs[] = {{256, 128}, {128, 256}, {128, 128}};
-    double best = -1.0;
+// The native kernel's tiles and their modelled times: a round of one-per-CU
+// tiles costs stages (64 elements) x (stage + occ x the share of CUs busy) +
+// round; the 64 x 64 tile (two per CU) goes by tiles per CU instead.  Fitted to
+// forced-configuration times (us; 256 x 128, 128 x 128, 64 x 128, 64 x 64): 512 x
+// 4096 -> 1536 -, 29.8, 21.7, 16.4; 512 x 1536 -> 1536 -, 13.3, 10.3, 7.8; 1000 x
+// 3072 -> 1536 -, 24.3, 18.2, 20.6; 1560 x 1536 -> 1536 19.7, 13.7, 19.9, 17.3;
+// 880 x 3072 -> 3072 34.3, 23.2, 33.2, 30.3; 4680 x 1536 -> 1536 23.1, 28.5, 39.3,
+// 37.3; 4680 x 64 -> 1536 6.7, 9.1, 13.3, 10.4.
+struct Bf16Cfg {
+    int bm, bn;
+    double stage, occ, round;
+};
+constexpr Bf16Cfg kBf16[] = {
+    {256, 128, 0.55, 0.25, 5.0}, {128, 256, 0.55, 0.25, 5.0}, {128, 128, 0.43, 0.0, 3.5}, {64, 128, 0.29, 0.0, 3.4}, {64, 64, 0.21, 0.0, 1.2},
+};
+
+int bf16_pick(int num_cu, size_t M, size_t N, size_t K, double *us) {
     int pick = 0;
-    for (int i = 0; i < 3; i++) {
-        const size_t tiles = ((M + cfgs[i].bm - 1) / cfgs[i].bm) * ((N + cfgs[i].bn - 1) / cfgs[i].bn);
-        const size_t rounds = (tiles + num_cu - 1) / num_cu;
-        const double eff = (double)M * N / ((double)rounds * num_cu * cfgs[i].bm * cfgs[i].bn);
-        if (eff > best * 1.0001) {
-            best = eff;
+    double best = 0.0;
+    const double st = (double)(K / BKE);
+    for (int i = 0; i < 5; i++) {
+        const Bf16Cfg &c = kBf16[i];
+        const size_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn), rounds = (tiles + num_cu - 1) / num_cu;
+        const double fill = (double)tiles / num_cu;
+        const double t = c.bm * c.bn == 64 * 64 ? std::max(1.0, fill) * (st * c.stage + c.round) + 1.6
+                                               : (double)rounds * (st * (c.stage + c.occ * std::min(1.0, fill)) + c.round);
+        if (i == 0 || t < best * 0.9999) {  // the larger tile on ties
+            best = t;
             pick = i;
         }
     }
+    *us = best;
+    return pick;
+}
+
+}  // namespace
+
+double gemm_bf16_cost_us(int num_cu, size_t M, size_t N, size_t K) {
+    double us;
+    bf16_pick(num_cu, M, N, K, &us);
+    return us;
+}
+
+void launch_gemm_bf16(hipStream_t s, int num_cu, const uint16_t *x, const uint16_t *w, const float *bias, int act,
+                      void *y, int y_dtype, size_t M, size_t N, size_t K) {
+    double us;
     const int m = (int)M, n = (int)N, k = (int)K;
-    switch (pick) {
+    switch (bf16_pick(num_cu, M, N, K, &us)) {
         case 0: launch_bf16_cfg<256, 128, 4, 2, 3>(s, x, w, bias, act, y, y_dtype, m, n, k); break;
         case 1: launch_bf16_cfg<128, 256, 2, 4, 3>(s, x, w, bias, act, y, y_dtype, m, n, k); break;
-        default: launch_bf16_cfg<128, 128, 2, 2, 3>(s, x, w, bias, act, y, y_dtype, m, n, k); break;
+        case 2: launch_bf16_cfg<128, 128, 2, 2, 3>(s, x, w, bias, act, y, y_dtype, m, n, k); break;
+        case 3: launch_bf16_cfg<64, 128, 2, 2, 4>(s, x, w, bias, act, y, y_dtype, m, n, k); break;
+        default: launch_bf16_cfg<64, 64, 2, 2, 4>(s, x, w, bias, act, y, y_dtype, m, n, k); break;
     }
 }
 
