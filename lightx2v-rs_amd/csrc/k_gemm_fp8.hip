@@ -1363,7 +1363,13 @@ __global__ __launch_bounds__(512, 1) void k_gemm_fp8_ov(const uint8_t *__restric
 // Constraints (host): K % 64 == 0, K / 64 >= 4, N % 256 == 0, M N sizeof(TY)
 // < 2^31; bf16 or MX e4m3 output; per-token activations, per-channel weight
 // scales; no residual mode.
-template <int BKB, int ACT, typename TY>
+//
+// BF: the same kernel over bf16 rows (A and B hold K / 2 elements a row, K
+// counts bytes; sa and sb unused).  A 64-byte slice is then two 32x32x16 bf16
+// MFMAs of half the length where fp8 has one, so the balance of LDS reads,
+// loads and matrix cycles is the same; lane half h reads chunk 2 k + h of
+// 16-element step k, the K order (and so the sums) of k_gemm_bf16_dma.
+template <int BKB, int ACT, typename TY, bool BF = false>
 __global__ __launch_bounds__(256, 1) void k_gemm_fp8_w4(const uint8_t *__restrict__ A, const float *__restrict__ sa,
                                                        const uint8_t *__restrict__ B, const float *__restrict__ sb,
                                                        const float *__restrict__ bias, TY *__restrict__ Y, int M,
@@ -1444,13 +1450,13 @@ __global__ __launch_bounds__(256, 1) void k_gemm_fp8_w4(const uint8_t *__restric
     // scales / channel scales / bias into the sc set of its parity (a null
     // bias reads zeros); every other ninth load goes to the dummy slot.
     auto ninth = [&]() {
-        const bool ops = is_kt == 0 && is_i < my_n && wid_u < 3;
+        const bool ops = is_kt == 0 && is_i < my_n && (BF ? wid_u == 2 : wid_u < 3);
         if (ops) {
             const uint32_t dst = sc_at + (uint32_t)(is_i & 1) * NV * 4u;
-            if (wid_u == 0)
+            if (!BF && wid_u == 0)
                 dma16_at(make_rsrc(sa + is_m0, __builtin_amdgcn_readfirstlane((uint32_t)(M - is_m0) * 4u)), dst,
                          (uint32_t)lane * 16u);
-            else if (wid_u == 1)
+            else if (!BF && wid_u == 1)
                 dma16_at(make_rsrc(sb + is_n0, __builtin_amdgcn_readfirstlane((uint32_t)(N - is_n0) * 4u)),
                          dst + BM * 4, (uint32_t)lane * 16u);
             else
@@ -1473,8 +1479,8 @@ __global__ __launch_bounds__(256, 1) void k_gemm_fp8_w4(const uint8_t *__restric
 
     // Fragments of one stage: the wave's TM activation row blocks and TN
     // weight row blocks, each 32 rows x 64 bytes as two 16-byte reads
-    // (lane half h: chunks 2 h and 2 h + 1 of the row).
-    const uint32_t frow = lane & 31, fhalf = (lane >> 5) * 2;
+    // (lane half h: chunks 2 h and 2 h + 1 of the row; BF: h and h + 2).
+    const uint32_t frow = lane & 31, fhalf = (lane >> 5) * (BF ? 1 : 2);
     struct Frag {
         u32x4 a[TM][2], b[TN][2];
     };
@@ -1482,7 +1488,7 @@ __global__ __launch_bounds__(256, 1) void k_gemm_fp8_w4(const uint8_t *__restric
     auto read_one = [&](int buf, int kk, Frag &f, int m) {
         const uint8_t *st = smem + buf * STAGE;
         const int fi = m >> 1, h = m & 1;
-        const uint32_t c = (uint32_t)kk * 4 + fhalf + (uint32_t)h;
+        const uint32_t c = (uint32_t)kk * 4 + fhalf + (uint32_t)(BF ? 2 * h : h);
         if (fi < TM) {
             const uint32_t row = wm * WM + fi * 32 + frow;
             f.a[fi][h] = *(const u32x4 *)(st + ((row * BKB + (dma_slot<BKB>(row, c) << 4)) & AMASK));
@@ -1510,7 +1516,16 @@ __global__ __launch_bounds__(256, 1) void k_gemm_fp8_w4(const uint8_t *__restric
     auto step = [&](auto FIRST, auto RD, auto L0, auto L1, const Frag &fc, Frag &fn, int rbuf, int rkk, int dbuf) {
         static_for<TN * TM>([&](auto JI) {
             constexpr int m = decltype(JI)::value, j = m / TM, i = m % TM;
-            if constexpr (decltype(FIRST)::value)
+            if constexpr (BF)
+                static_for<2>([&](auto QI) {  // the slice's first 16-element step on every block, then its second
+                    constexpr int q = 2 * m + decltype(QI)::value, h = q / (TN * TM), bj = q / TM % TN, bi = q % TM;
+                    const bf16x8 wf = __builtin_bit_cast(bf16x8, fc.b[bj][h]), xf = __builtin_bit_cast(bf16x8, fc.a[bi][h]);
+                    if constexpr (decltype(FIRST)::value && h == 0)
+                        acc[bj][bi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, xf, (f32x16){}, 0, 0, 0);
+                    else
+                        acc[bj][bi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, xf, acc[bj][bi], 0, 0, 0);
+                });
+            else if constexpr (decltype(FIRST)::value)
                 acc[j][i] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(as8(fc.b[j]), as8(fc.a[i]), (f32x16){}, 0, 0,
                                                                             0, 0, 0, 0);
             else
@@ -1540,17 +1555,21 @@ __global__ __launch_bounds__(256, 1) void k_gemm_fp8_w4(const uint8_t *__restric
 #pragma unroll
             for (int g = 0; g < 4; g++) {
                 const int c = cb + 8 * g + 4 * hf;
-                cs[g] = *(const f32x4 *)(sct + BM + c);
+                if constexpr (!BF) cs[g] = *(const f32x4 *)(sct + BM + c);
                 bs[g] = *(const f32x4 *)(sct + BM + BN + c);
             }
             static_for<TM>([&](auto I) {
                 constexpr int i = decltype(I)::value;
-                const float tsc = sct[wm * WM + i * 32 + l32];
+                const float tsc = BF ? 1.0f : sct[wm * WM + i * 32 + l32];
                 float v[16];
                 float amax = 0.0f;
 #pragma unroll
                 for (int e = 0; e < 16; e++) {
-                    float t = acc[j][i][e] * tsc * cs[e / 4][e % 4] + bs[e / 4][e % 4];
+                    float t;
+                    if constexpr (BF)
+                        t = acc[j][i][e] + bs[e / 4][e % 4];
+                    else
+                        t = acc[j][i][e] * tsc * cs[e / 4][e % 4] + bs[e / 4][e % 4];
                     if constexpr (GELU) t = gelu_tanh_fast(t);
                     v[e] = t;
                     if constexpr (EB == 1) amax = fmaxf(amax, fabsf(t));
@@ -2001,6 +2020,31 @@ void launch_w4(hipStream_t s, int num_cu, const uint8_t *a, const float *sa, con
     }
 #undef LX2V_W4
 }
+
+}  // namespace
+
+bool gemm_bf16_w4_supported(size_t M, size_t N, size_t K, int y_dtype) {
+    return y_dtype == LX2V_DTYPE_BF16 && N % 256 == 0 && K % 64 == 0 && K >= 128 && M * N * 2 < (1ull << 31) &&
+           gemm_bf16_supported(M, N, K);
+}
+
+void launch_gemm_bf16_w4(hipStream_t s, int num_cu, const uint16_t *x, const uint16_t *w, const float *bias, int act,
+                         uint16_t *y, int M, int N, int K) {
+    const int tiles_m = (M + 255) / 256, tiles_n = N / 256, nt = tiles_m * tiles_n;
+    int g = nt < num_cu ? nt : num_cu;
+    if (g < nt && g >= 8) g = g / 8 * 8;
+    const uint8_t *a = (const uint8_t *)x, *b = (const uint8_t *)w;
+#define LX2V_W4(ACTV)                                                                                            \
+    hipLaunchKernelGGL((k_gemm_fp8_w4<128, ACTV, uint16_t, true>), dim3(g), dim3(256), 0, s, a, nullptr, b, nullptr, \
+                       bias, y, M, N, 2 * K, tiles_m, tiles_n, nullptr, 0)
+    if (act == LX2V_ACT_GELU_TANH)
+        LX2V_W4(LX2V_ACT_GELU_TANH);
+    else
+        LX2V_W4(LX2V_ACT_NONE);
+#undef LX2V_W4
+}
+
+namespace {
 
 // Direct-to-LDS configurations: tile (activation rows x channels), wave
 // grid, K bytes per stage, stages.

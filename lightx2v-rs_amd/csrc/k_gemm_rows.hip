@@ -332,6 +332,8 @@ dim3 rows_grid(size_t M, size_t N, int mb) {
 // LIGHTX2V_HIP_ROWS=<n> takes it for every call of up to n rows instead.
 bool gemm_rows_chosen(RowsKind kind, int num_cu, size_t M, size_t N, size_t K, double tile_us) {
     if (K % 64 || N == 0 || M == 0) return false;
+    // 32-bit offsets into the rows as they are (the tiles read f32 ones as bf16)
+    if (kind == RowsKind::F32Act && M * K * 4 >= (1ull << 31)) return false;
     // a pinned tile configuration stays the tile kernels'
     for (const char *pin : {"LIGHTX2V_HIP_FP8_CFG", "LIGHTX2V_HIP_W16_CFG"}) {
         const char *e = getenv(pin);

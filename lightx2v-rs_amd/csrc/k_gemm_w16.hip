@@ -909,17 +909,92 @@ int plan_gemm_w16_dma(int num_cu, size_t M, size_t N) {
     return pick;
 }
 
-// 256 x 128 and 128 x 256 tiles cost about 0.88 us per 64-element stage, the
-// 256 x 256 one 1.55 (M 128 .. 1560, K 512 .. 14336: within 15%).
-double gemm_w16_dma_cost_us(int num_cu, size_t M, size_t N, size_t K) {
+// A 64-element stage of the 256 x 128 and 128 x 256 tiles costs 0.86 us plus
+// what the dequantization adds with every CU busy (power and LDS), of the 256 x
+// 256 one about twice that (M 300 .. 4680, K 512 .. 14336: within 15%).
+double gemm_w16_dma_cost_us(int num_cu, const lx2v_hip_weight *w, size_t M) {
+    const size_t N = w->rows, K = w->cols;
     const DmaCfg &c = kDmaW16[plan_gemm_w16_dma(num_cu, M, N)];
+    const bool q4 = w->fmt == LX2V_WFMT_Q4, big = c.bm * c.bn > 256 * 128;
     const size_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
-    return (double)((tiles + num_cu - 1) / num_cu) * ((double)K / 64 * (c.bm * c.bn > 256 * 128 ? 1.55 : 0.88) + 4.0);
+    const double busy = std::min(1.0, (double)tiles / num_cu);
+    const double stage = big ? (q4 ? 1.45 + 0.25 * busy : 1.50 + 0.30 * busy) : 0.86 + (q4 ? 0.16 : 0.25) * busy;
+    return (double)((tiles + num_cu - 1) / num_cu) * ((double)K / 64 * stage + (big ? 10.0 : 3.0 + 4.0 * busy));
 }
 
 void launch_gemm_w16_dma(hipStream_t s, int cfg, const uint16_t *x, const lx2v_hip_weight *w, const float *bias,
                          int act, void *y, int y_dtype, size_t M) {
     launch_dma_idx(cfg, s, x, w, bias, act, y, y_dtype, (int)M);
+}
+
+namespace {
+
+// A weight's bf16 values, [N, K]: the values the GEMM's own dequantization
+// gives.  Bound by the 2 bytes written per element; a thread takes 16
+// elements, so a wave reads 1 KB of codes and writes 2 KB in a row.
+template <int WF>
+__global__ __launch_bounds__(256) void k_w16_expand(const uint8_t *__restrict__ codes, const float *__restrict__ scales,
+                                                    const float *__restrict__ zeros, uint16_t *__restrict__ out,
+                                                    uint32_t units, uint32_t ug) {
+    constexpr bool Q4 = WF == LX2V_WFMT_Q4 || WF == kWfmtQ4Sym;
+    const uint32_t u = blockIdx.x * 256u + threadIdx.x;  // 16 elements of one row, ug units to a scale
+    if (u >= units) return;
+    u32x4 c;
+    if constexpr (Q4) {
+        const u32x2 h = *(const u32x2 *)(codes + (size_t)u * 8);
+        c = (u32x4){h.x, h.y, 0u, 0u};
+    } else {
+        c = *(const u32x4 *)(codes + (size_t)u * 16);
+    }
+    const uint32_t g = u / ug;  // K % group == 0, so groups follow one another across rows
+    uint32_t o[8];
+    unit_dequant<WF>(c, scales[g], WF == LX2V_WFMT_Q4 ? zeros[g] : 0.0f, o);
+    u32x4 *p = (u32x4 *)(out + (size_t)u * 16);
+    p[0] = (u32x4){o[0], o[1], o[2], o[3]};
+    p[1] = (u32x4){o[4], o[5], o[6], o[7]};
+}
+
+}  // namespace
+
+// Dequantizing inside the GEMM costs every stage of every tile row, and that
+// kernel's tiles are large; written out once, the weight goes through tiles of
+// every size with nothing but loads and MFMAs in their stages.  Inside ->
+// written out (us, both launches; Q8 / Q4, bf16 in and out): 4680 x 1536 -> 8960
+// 162 -> 133 / 151 -> 132, 4680 x 8960 -> 1536 159 -> 129 / 139 -> 125, 300 x
+// 8960 -> 1536 127 -> 45 / 120 -> 45, 300 x 1536 -> 1536 23 -> 15, 4680 x 3072
+// -> 14336 472 -> 382.  A short GEMM over a wide weight does not repay the pass:
+// 600 x 1536 -> 4608 25.1 / 27.3, 300 x 3072 -> 14336 54 / 65, 1560 x 1536 -> 8960
+// 57 / 59, 4680 x 1536 -> 1536 32.6 / 33.3.  The pass and the cold read of what
+// it wrote take 7.5 us + 0.48 us per million weights; 3.5 us more is asked so
+// that the models' errors do not pick the slower side.  Weights up to 128 MB
+// written out bound the workspace.
+// LIGHTX2V_HIP_W16_EXPAND=0 / 1 pins the choice for calls that both sides take.
+bool w16_expand_chosen(int num_cu, const lx2v_hip_weight *w, size_t M, int y_dtype) {
+    const size_t N = w->rows, K = w->cols;
+    if (!gemm_w16_dma_supported(w, M) || !gemm_bf16_supported(M, N, K) || N * K * 2 > (128u << 20)) return false;
+    const char *cfg = getenv("LIGHTX2V_HIP_W16_CFG");
+    if (cfg && *cfg && atoi(cfg) >= 0) return false;  // a pinned tile dequantizes inside
+    const char *e = getenv("LIGHTX2V_HIP_W16_EXPAND");
+    if (e && *e) return atoi(e) != 0;
+    return 7.5 + (double)(N * K) * 0.48e-6 + gemm_bf16_cost_us(num_cu, M, N, K, y_dtype) + 3.5 < gemm_w16_dma_cost_us(num_cu, w, M);
+}
+
+void launch_w16_expand(hipStream_t s, const lx2v_hip_weight *w, uint16_t *out) {
+    const uint32_t units = (uint32_t)(w->rows * w->cols / 16), ug = (uint32_t)(w->group / 16);
+    const dim3 grid((units + 255) / 256), block(256);
+    const uint8_t *c = (const uint8_t *)w->codes;
+#define LX2V_EXPAND(WF) hipLaunchKernelGGL((k_w16_expand<WF>), grid, block, 0, s, c, w->scales, w->zeros, out, units, ug)
+    switch (w->fmt) {
+        case LX2V_WFMT_Q8: LX2V_EXPAND(LX2V_WFMT_Q8); break;
+        case LX2V_WFMT_Q4:
+            if (w->zero8)
+                LX2V_EXPAND(kWfmtQ4Sym);
+            else
+                LX2V_EXPAND(LX2V_WFMT_Q4);
+            break;
+        default: LX2V_EXPAND(LX2V_WFMT_FP8); break;
+    }
+#undef LX2V_EXPAND
 }
 
 bool gemm_bf16_supported(size_t M, size_t N, size_t K) {
@@ -945,7 +1020,7 @@ constexpr Bf16Cfg kBf16[] = {
     {256, 128, 0.55, 0.25, 5.0}, {128, 256, 0.55, 0.25, 5.0}, {128, 128, 0.43, 0.0, 3.5}, {64, 128, 0.29, 0.0, 3.4}, {64, 64, 0.21, 0.0, 1.2},
 };
 
-int bf16_pick(int num_cu, size_t M, size_t N, size_t K, double *us) {
+int bf16_pick(int num_cu, size_t M, size_t N, size_t K, int y_dtype, double *us) {
     int pick = 0;
     double best = 0.0;
     const double st = (double)(K / BKE);
@@ -960,15 +1035,32 @@ int bf16_pick(int num_cu, size_t M, size_t N, size_t K, double *us) {
             pick = i;
         }
     }
+    if (gemm_bf16_w4_supported(M, N, K, y_dtype)) {
+        // The persistent 256 x 256 tile: 1.02 us a stage (0.85 of MFMA) up to
+        // half the CUs, 1.38 with all, 7.8 a round.  256 x 128 / this: 4680 x 1536
+        // -> 8960 142 / 116, 4680 x 14336 -> 3072 368 / 314, 4680 x 3072 -> 14336
+        // 386 / 355, 2640 x 1536 -> 4608 47 / 39; 4680 x 8960 -> 1536 117 / 151.
+        const size_t tiles = (M + 255) / 256 * (N / 256), full = tiles / num_cu;
+        const double last = (double)(tiles % num_cu) / num_cu, crowd = std::min(1.0, std::max(0.0, (last - 0.5) / 0.4));
+        const double t = (double)full * (st * 1.38 + 7.8) + (last > 0.0 ? st * (1.02 + 0.36 * crowd) + 7.8 : 0.0);
+        if (t < best * 0.9999) {
+            best = t;
+            pick = 5;
+        }
+    }
+    if (const char *e = getenv("LIGHTX2V_HIP_BF16_CFG")) {  // pins a tile that takes the call (tests)
+        const int i = atoi(e);
+        if (*e && i >= 0 && (i < 5 || (i == 5 && gemm_bf16_w4_supported(M, N, K, y_dtype)))) pick = i;
+    }
     *us = best;
     return pick;
 }
 
 }  // namespace
 
-double gemm_bf16_cost_us(int num_cu, size_t M, size_t N, size_t K) {
+double gemm_bf16_cost_us(int num_cu, size_t M, size_t N, size_t K, int y_dtype) {
     double us;
-    bf16_pick(num_cu, M, N, K, &us);
+    bf16_pick(num_cu, M, N, K, y_dtype, &us);
     return us;
 }
 
@@ -976,11 +1068,12 @@ void launch_gemm_bf16(hipStream_t s, int num_cu, const uint16_t *x, const uint16
                       void *y, int y_dtype, size_t M, size_t N, size_t K) {
     double us;
     const int m = (int)M, n = (int)N, k = (int)K;
-    switch (bf16_pick(num_cu, M, N, K, &us)) {
+    switch (bf16_pick(num_cu, M, N, K, y_dtype, &us)) {
         case 0: launch_bf16_cfg<256, 128, 4, 2, 3>(s, x, w, bias, act, y, y_dtype, m, n, k); break;
         case 1: launch_bf16_cfg<128, 256, 2, 4, 3>(s, x, w, bias, act, y, y_dtype, m, n, k); break;
         case 2: launch_bf16_cfg<128, 128, 2, 2, 3>(s, x, w, bias, act, y, y_dtype, m, n, k); break;
         case 3: launch_bf16_cfg<64, 128, 2, 2, 4>(s, x, w, bias, act, y, y_dtype, m, n, k); break;
+        case 5: launch_gemm_bf16_w4(s, num_cu, x, w, bias, act, (uint16_t *)y, m, n, k); break;
         default: launch_bf16_cfg<64, 64, 2, 2, 4>(s, x, w, bias, act, y, y_dtype, m, n, k); break;
     }
 }

@@ -337,7 +337,7 @@ int lx2v_hip_destroy(lx2v_hip_ctx *ctx) {
     for (auto e : ctx->prof.pool) (void)hipEventDestroy(e);
     for (auto &r : ctx->prof.open_regions) (void)hipEventDestroy(r.second);
     if (ctx->ws) (void)hipFree(ctx->ws);
-    for (lx2v::Stage *x : {&ctx->stage, &ctx->mask, &ctx->kv_spare, &ctx->resid, &ctx->attn, &ctx->splitk})
+    for (lx2v::Stage *x : {&ctx->stage, &ctx->mask, &ctx->kv_spare, &ctx->resid, &ctx->attn, &ctx->wexp, &ctx->splitk})
         if (x->ptr) (void)hipFree(x->ptr);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -2005,7 +2005,7 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
     else if (native_bf16 || gemm_w16_dma_supported(w, rows))
         few = gemm_rows_chosen(x->dtype == LX2V_DTYPE_F32 ? RowsKind::F32Act : native_bf16 ? RowsKind::Native : RowsKind::W16,
                                ctx->num_cu, rows, N, K,
-                               (native_bf16 ? gemm_bf16_cost_us(ctx->num_cu, rows, N, K) : gemm_w16_dma_cost_us(ctx->num_cu, rows, N, K)) +
+                               (native_bf16 ? gemm_bf16_cost_us(ctx->num_cu, rows, N, K, y->dtype) : gemm_w16_dma_cost_us(ctx->num_cu, w, rows)) +
                                    (x->dtype == LX2V_DTYPE_F32 ? 2.5 : 0.0));  // the tiles' pass that rounds f32 rows to bf16
     if (few) plan.splits = 1;
     // Workspaces, each piece 256-byte aligned: a bf16 bias's f32 copy; the
@@ -2143,6 +2143,24 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
     if (gemm_w16_dma_supported(w, rows)) {
         const uint16_t *xb;
         if (int rc = bf16_x(&xb)) return rc;
+        // Many rows: the weight's bf16 values written out once, then the bf16
+        // GEMM on them (the same products in the same order).  Not in a
+        // graph, which would hold the workspace, nor where nothing may be
+        // allocated; without the memory the tiles below take the call.
+        if (!scr && !ctx->capturing && w16_expand_chosen(ctx->num_cu, w, rows, y->dtype)) {
+            if (ensure(ctx, &ctx->wexp.ptr, &ctx->wexp.bytes, N * K * 2, "weight workspace alloc") == LX2V_OK) {
+                uint16_t *wx = (uint16_t *)ctx->wexp.ptr;
+                if (int rc = run(ctx, "w16_expand", [&] { launch_w16_expand(ctx->stream, w, wx); })) return rc;
+                char xname[40];
+                snprintf(xname, sizeof xname, "%s.bf16", name);
+                if (int rc = run(ctx, xname, [&] {
+                        launch_gemm_bf16(ctx->stream, ctx->num_cu, xb, wx, bp, act, yp, y->dtype, rows, N, K);
+                    }))
+                    return rc;
+                return ok();
+            }
+            (void)hipGetLastError();
+        }
         const int cfg = plan_gemm_w16_dma(ctx->num_cu, rows, N);
         char pname[40];  // e.g. "gemm_w16_q8.c2": the tile configuration
         snprintf(pname, sizeof pname, "%s.c%d", name, cfg);

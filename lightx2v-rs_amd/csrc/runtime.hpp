@@ -151,6 +151,7 @@ struct lx2v_hip_ctx {
     lx2v::Stage kv_spare;  // the MemRoPE update's output layout, swapped with the cache it updates
     lx2v::Stage resid;     // linear_residual's output where the add cannot ride in the GEMM
     lx2v::Stage attn;      // split attention's partial sums (attention_split)
+    lx2v::Stage wexp;      // a Q8 / Q4 / FP8 weight's bf16 values for one call (w16_expand_chosen)
     lx2v::Stage splitk;    // split-K fp8 GEMM partial sums (Fp8Plan::splits)
     // The no-alloc entry point's hold on the device scratch: recorded after
     // each of its calls (and each launch of a graph that holds such calls);
@@ -357,14 +358,23 @@ void launch_gemm_w16(hipStream_t s, int num_cu, const void *x, int x_dtype,
                      size_t M);
 bool gemm_w16_dma_supported(const lx2v_hip_weight *w, size_t M);
 int plan_gemm_w16_dma(int num_cu, size_t M, size_t N);
-double gemm_w16_dma_cost_us(int num_cu, size_t M, size_t N, size_t K);  // modelled time of its choice
+double gemm_w16_dma_cost_us(int num_cu, const lx2v_hip_weight *w, size_t M);  // modelled time of its choice
 void launch_gemm_w16_dma(hipStream_t s, int cfg, const uint16_t *x, const lx2v_hip_weight *w, const float *bias,
                          int act, void *y, int y_dtype, size_t M);
+// The weight's bf16 values written out for launch_gemm_bf16, and whether that
+// pass and GEMM beat dequantizing inside launch_gemm_w16_dma.
+bool w16_expand_chosen(int num_cu, const lx2v_hip_weight *w, size_t M, int y_dtype);
+void launch_w16_expand(hipStream_t s, const lx2v_hip_weight *w, uint16_t *out);
 // bf16 x bf16 (native f32 weights through their bf16 copy): X [M, K] and
 // W [N, K] bf16, K % 64 == 0.
 bool gemm_bf16_supported(size_t M, size_t N, size_t K);
-double gemm_bf16_cost_us(int num_cu, size_t M, size_t N, size_t K);  // modelled time of launch_gemm_bf16's choice
+double gemm_bf16_cost_us(int num_cu, size_t M, size_t N, size_t K, int y_dtype);  // modelled time of launch_gemm_bf16's choice
 void launch_gemm_bf16(hipStream_t s, int num_cu, const uint16_t *x, const uint16_t *w, const float *bias, int act,
                       void *y, int y_dtype, size_t M, size_t N, size_t K);
+// k_gemm_fp8.hip: the persistent 256 x 256 tile over bf16 rows, one of
+// launch_gemm_bf16's choices (bf16 output, N % 256 == 0).
+bool gemm_bf16_w4_supported(size_t M, size_t N, size_t K, int y_dtype);
+void launch_gemm_bf16_w4(hipStream_t s, int num_cu, const uint16_t *x, const uint16_t *w, const float *bias, int act,
+                         uint16_t *y, int M, int N, int K);
 
 }  // namespace lx2v

@@ -1,0 +1,82 @@
+"""Two ways to the same sums on the bf16 MFMA: the 256 x 256 persistent tile
+against the 256 x 128 one (LIGHTX2V_HIP_BF16_CFG), and a Q8 / Q4 / FP8 weight
+written out as bf16 first against dequantization inside the GEMM
+(LIGHTX2V_HIP_W16_EXPAND).  Both sides contract the same bf16 values in the
+same 16-element steps in the same order, so outputs agree bit for bit."""
+
+import numpy as np
+import pytest
+
+import lightx2v_hip as H
+import oracle as O
+from helpers import W16_TIGHT, assert_close, normal, oracle_w16, u32
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(be, x, w, b, act, M, N, ydt):
+    y = be.alloc((M + 1) * N, ydt)
+    be.write(y, np.full((M + 1) * N, np.nan, np.float32))
+    be.profile_reset()
+    be.profile_enable(True)
+    try:
+        be.linear(x, 1, M, w, b, act, y, 0)
+        names = list(be.profile_stats())
+    finally:
+        be.profile_enable(False)
+        be.profile_reset()
+    v = be.download(y).reshape(M + 1, N)
+    assert np.isnan(v[M]).all() and not np.isnan(v[:M]).any()
+    return v[:M], names
+
+
+# K of two, three and many stages; one row, tile edges, more tiles than CUs
+@pytest.mark.parametrize("M,K,N", [(1, 128, 256), (255, 192, 512), (257, 1536, 256), (2500, 128, 7936), (600, 320, 768)])
+@pytest.mark.parametrize("act", [H.ACT_NONE, H.ACT_GELU_TANH])
+def test_bf16_persistent_tile_equals_tiles(be, monkeypatch, act, M, K, N):
+    monkeypatch.setenv("LIGHTX2V_HIP_ROWS", "0")
+    wf, xf, bf = normal(4401 + N, N * K, 0.02), normal(4402, (M + 1) * K), normal(4403, N, 0.01)
+    w, x, b = be.weight(wf, N, K), be.alloc((M + 1) * K, H.DTYPE_BF16), be.upload(bf)
+    be.write(x, xf)
+    out = []
+    for cfg in ("0", "5"):
+        monkeypatch.setenv("LIGHTX2V_HIP_BF16_CFG", cfg)
+        out.append(_run(be, x, w, b if M != 257 else None, act, M, N, H.DTYPE_BF16)[0])
+    assert np.array_equal(u32(out[0]), u32(out[1]))
+    p = np.unique(np.append(np.arange(0, M, 97), M - 1))
+    ref = oracle_w16(O.bf16_round(xf).reshape(M + 1, K)[1:][p], wf.reshape(N, K), bf if M != 257 else None, act)
+    assert_close(out[1][p], ref, W16_TIGHT[0] + 2.0**-8, W16_TIGHT[1] + 2.0**-7 * np.abs(ref).max(), what="vs oracle")
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 64, 33), (300, 192, 96), (257, 1536, 512)])
+@pytest.mark.parametrize("xdt", [H.DTYPE_F32, H.DTYPE_BF16])
+@pytest.mark.parametrize("fmt", ["q8_32", "q8_64", "q8_16", "q4_32", "q4_zeros_64", "fp8_64"])
+def test_expanded_weight_equals_dequantized(be, monkeypatch, fmt, xdt, M, K, N):
+    monkeypatch.setenv("LIGHTX2V_HIP_ROWS", "0")
+    g, wf = int(fmt.split("_")[-1]), normal(4501 + N + K, N * K, 0.02).reshape(N, K)
+    if fmt.startswith("q8"):
+        q, s = O.q8_quantize(wf, N, K, g)
+        w = be.weight_q8(q, s, N, K, g)
+    elif fmt.startswith("q4"):
+        c, s, z = O.q4_quantize_sym(wf, N, K, g)
+        if "zeros" in fmt:
+            z = z + (np.arange(z.size, dtype=np.float32).reshape(z.shape) % 3 - 1) * np.float32(0.5)
+        w = be.weight_q4(O.q4_pack(c), s, z, N, K, g, packed=True)
+    else:
+        q, s = O.fp8_quantize(wf, N, K, g, True)
+        w = be.weight_fp8(q, s, N, K, g)
+    x, b = be.alloc((M + 1) * K, xdt), be.upload(normal(4503, N, 0.01))
+    be.write(x, normal(4502, (M + 1) * K))
+    if fmt == "fp8_64":
+        be.set_fp8_act(H.FP8_ACT_BF16)
+    try:
+        for ydt in (H.DTYPE_BF16, H.DTYPE_F32):
+            out = []
+            for e in ("0", "1"):
+                monkeypatch.setenv("LIGHTX2V_HIP_W16_EXPAND", e)
+                v, names = _run(be, x, w, b, H.ACT_GELU_TANH, M, N, ydt)
+                assert ("w16_expand" in names) == (e == "1"), names
+                out.append(v)
+            assert np.array_equal(u32(out[0]), u32(out[1]))
+    finally:
+        be.set_fp8_act(H.FP8_ACT_E4M3)
