@@ -321,6 +321,11 @@ dim3 rows_grid(size_t M, size_t N, int mb) {
 
 }  // namespace
 
+size_t gemm_rows_limit(RowsKind kind) {
+    const char *e = getenv("LIGHTX2V_HIP_ROWS");
+    return e && *e ? (size_t)std::max(0, atoi(e)) : kind == RowsKind::Fp8 ? 64 : 256;
+}
+
 // The modelled time: a wave's share of the 128-element steps, each slower with
 // the rows it loads, times the workgroups a CU runs where they outnumber the
 // CUs.  Fitted at 1536 -> 1536, 14336 -> 1536 and 3072 -> 14336 (M 1 .. 64; us,
@@ -340,8 +345,8 @@ bool gemm_rows_chosen(RowsKind kind, int num_cu, size_t M, size_t N, size_t K, d
         if (e && *e && atoi(e) >= 0) return false;
     }
     const char *e = getenv("LIGHTX2V_HIP_ROWS");
-    if (e && *e) return M <= (size_t)std::max(0, atoi(e));
-    if (M > (kind == RowsKind::Fp8 ? 64 : 256)) return false;
+    if (M > gemm_rows_limit(kind)) return false;
+    if (e && *e) return true;
     struct Step {
         double us, row_us, crowd;
     };

@@ -1924,10 +1924,12 @@ static int act_quant_into_ws(lx2v_hip_ctx *ctx, const void *x, int dtype, size_t
 // Whether the few-rows kernel takes an FP8 linear, decided against the plan
 // linear itself would make (linear_residual asks the same question, so that
 // both sum in the same order).
+// known: that plan, if the caller has made it.
 static bool few_rows_fp8(const lx2v_hip_ctx *ctx, size_t rows, const lx2v_hip_weight *w, bool x_mx, bool y_mx, bool grouped,
-                         int y_dtype, int act) {
+                         int y_dtype, int act, const Fp8Plan *known = nullptr) {
     const size_t N = w->rows, K = w->cols;
-    const Fp8Plan p = plan_gemm_fp8(ctx->num_cu, rows, N, K, x_mx || y_mx, x_mx, grouped, y_dtype, act, false, true);
+    if (rows > gemm_rows_limit(RowsKind::Fp8)) return false;
+    const Fp8Plan p = known ? *known : plan_gemm_fp8(ctx->num_cu, rows, N, K, x_mx || y_mx, x_mx, grouped, y_dtype, act, false, true);
     if (p.splits > 1 && p.cost_us == 0.0) return false;  // a forced split
     // (group-128 and MX stages of the few-tile configurations run slower than modelled)
     return gemm_rows_chosen(RowsKind::Fp8, ctx->num_cu, rows, N, K, p.cost_us * (grouped ? 1.4 : x_mx ? 1.2 : 1.0));
@@ -2001,8 +2003,8 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
     // Few rows: the kernels that read the weight once, on the same operands.
     bool few = false;
     if (e4m3_path)
-        few = fp8_mfma && few_rows_fp8(ctx, rows, w, x_mx, y_mx, fp8_grouped, y->dtype, act);
-    else if (native_bf16 || gemm_w16_dma_supported(w, rows))
+        few = fp8_mfma && few_rows_fp8(ctx, rows, w, x_mx, y_mx, fp8_grouped, y->dtype, act, gate ? nullptr : &plan);
+    else if (rows <= gemm_rows_limit(RowsKind::W16) && (native_bf16 || gemm_w16_dma_supported(w, rows)))
         few = gemm_rows_chosen(x->dtype == LX2V_DTYPE_F32 ? RowsKind::F32Act : native_bf16 ? RowsKind::Native : RowsKind::W16,
                                ctx->num_cu, rows, N, K,
                                (native_bf16 ? gemm_bf16_cost_us(ctx->num_cu, rows, N, K, y->dtype) : gemm_w16_dma_cost_us(ctx->num_cu, w, rows)) +

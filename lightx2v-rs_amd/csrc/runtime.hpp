@@ -341,6 +341,7 @@ void launch_gemm_fp8(hipStream_t s, int num_cu, const Fp8Plan &p, const uint8_t 
 // bf16 copy.  gemm_rows_chosen: whether it takes a call that would otherwise
 // cost tile_us on the tile kernels.
 enum class RowsKind { Fp8, W16, Native, F32Act };  // F32Act: f32 activations of the bf16 MFMA kinds
+size_t gemm_rows_limit(RowsKind kind);  // the most rows it is asked for (larger calls skip the models)
 bool gemm_rows_chosen(RowsKind kind, int num_cu, size_t M, size_t N, size_t K, double tile_us);
 void launch_gemm_rows_fp8(hipStream_t s, const uint8_t *x, const float *x_scale, const lx2v_hip_weight *w, bool grouped,
                           const float *bias, int act, void *y, int y_dtype, size_t M, const Fp8Mx &mx);
