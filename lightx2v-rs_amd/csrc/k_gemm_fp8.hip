@@ -290,11 +290,11 @@ __global__ __launch_bounds__(256, 1) void k_gemm_fp8(const uint8_t *__restrict__
 // (Fp8E4M3 with group 128, quant.rs:21, 425-429), BKB = 128 so that a stage
 // is exactly one scale group.  Wave 0 adds one DMA per stage: the stage's
 // BN channel ratios s_{kt-1} / s_kt from the weight's ratio table (row kt
-// of gsc, N floats a row; row 0 all ones).  Before the stage's first MFMA on
-// a block, the block's sums are multiplied by its channels' ratios, so the
-// accumulator always holds the sum in units of the current group's scale;
-// sb holds the last group's scales, which the epilogue applies as a
-// per-channel scale, and sa still scales each token.
+// of gsc, gratio_stride(N) floats a row; row 0 all ones).  Before the stage's
+// first MFMA on a block, the block's sums are multiplied by its channels'
+// ratios, so the accumulator always holds the sum in units of the current
+// group's scale; sb holds the last group's scales, which the epilogue applies
+// as a per-channel scale, and sa still scales each token.
 //
 // ACT: the epilogue activation (LX2V_ACT_*), a template parameter so that the
 // epilogue holds one copy of its staging code.
@@ -368,7 +368,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void k_gemm_fp8_dma(const uint
                                                                 : 0u));
     const auto rg_src = make_rsrc(
         GS ? (const uint8_t *)(gsc + n0) : A,
-        __builtin_amdgcn_readfirstlane(GS ? ((uint32_t)KT * (uint32_t)N - (uint32_t)n0) * 4u : 0u));
+        __builtin_amdgcn_readfirstlane(GS ? ((uint32_t)KT * (uint32_t)gratio_stride(N) - (uint32_t)n0) * 4u : 0u));
 
     // Load i of this wave covers tile rows [(i NW + wid) RPI, +RPI); lane l
     // fills slot l % CPR of row l / CPR.
@@ -399,11 +399,11 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void k_gemm_fp8_dma(const uint
     auto issue_scales = [&](int kt, int buf) {
         if constexpr (GS) {
             // lane l: the ratios of channels n0 + 4 l .. + 3 at stage kt; past
-            // the last channel the next row (or zeros at the end) is read, for
-            // channels that are never stored
+            // the last channel the row's padding and the next row (or zeros at
+            // the end) are read, for channels that are never stored
             if (wid_u == 0) {
                 const bool ok = kt < KT && lane < BN / 4;
-                dma16(rg_src, gsl + buf * GSL, ok ? (uint32_t)kt * (uint32_t)N * 4u + (uint32_t)lane * 16u : kOob);
+                dma16(rg_src, gsl + buf * GSL, ok ? (uint32_t)kt * (uint32_t)gratio_stride(N) * 4u + (uint32_t)lane * 16u : kOob);
             }
         }
         if constexpr (AM) {
@@ -781,7 +781,7 @@ __global__ __launch_bounds__(512, 1) void k_gemm_fp8_pt(const uint8_t *__restric
         rb_src = make_rsrc(B + (size_t)is_n0 * K, __builtin_amdgcn_readfirstlane((uint32_t)(N - is_n0) * (uint32_t)K));
         if constexpr (GS)
             rg_src = make_rsrc(gsc + is_n0, __builtin_amdgcn_readfirstlane(
-                                                ((uint32_t)KT * (uint32_t)N - (uint32_t)is_n0) * 4u));
+                                                ((uint32_t)KT * (uint32_t)gratio_stride(N) - (uint32_t)is_n0) * 4u));
     };
     set_issue_tile();
 
@@ -812,7 +812,7 @@ __global__ __launch_bounds__(512, 1) void k_gemm_fp8_pt(const uint8_t *__restric
         if constexpr (GS) {
             if (wid_u == 0) {
                 const bool ok = is_i < my_n && lane < BN / 4;
-                dma16(rg_src, gsl + buf * GSL, ok ? (uint32_t)is_kt * (uint32_t)N * 4u + (uint32_t)lane * 16u : kOob);
+                dma16(rg_src, gsl + buf * GSL, ok ? (uint32_t)is_kt * (uint32_t)gratio_stride(N) * 4u + (uint32_t)lane * 16u : kOob);
             }
         }
     };
@@ -1048,7 +1048,7 @@ __global__ __launch_bounds__(512, 1) void k_gemm_fp8_ov(const uint8_t *__restric
         rb_src = make_rsrc(B + (size_t)is_n0 * K, __builtin_amdgcn_readfirstlane((uint32_t)(N - is_n0) * (uint32_t)K));
         if constexpr (GS)
             rg_src = make_rsrc(gsc + is_n0, __builtin_amdgcn_readfirstlane(
-                                                ((uint32_t)KT * (uint32_t)N - (uint32_t)is_n0) * 4u));
+                                                ((uint32_t)KT * (uint32_t)gratio_stride(N) - (uint32_t)is_n0) * 4u));
     };
     set_issue_tile();
     const uint32_t lrow = (uint32_t)lane / CPR, lslot = (uint32_t)lane % CPR;
@@ -1081,7 +1081,7 @@ __global__ __launch_bounds__(512, 1) void k_gemm_fp8_ov(const uint8_t *__restric
             if (wid_u == 0) {
                 const bool ok = is_i < my_n && lane < BN / 4;
                 dma16_at(rg_src, gsl_at + (uint32_t)(buf * GSL),
-                         ok ? (uint32_t)is_kt * (uint32_t)N * 4u + (uint32_t)lane * 16u : kOob);
+                         ok ? (uint32_t)is_kt * (uint32_t)gratio_stride(N) * 4u + (uint32_t)lane * 16u : kOob);
             }
         }
     };
@@ -2191,8 +2191,7 @@ bool gemm_fp8_residual_ok(const Fp8Plan &p) {
 }
 
 bool gemm_fp8_grouped_supported(size_t M, size_t N, size_t K, size_t group) {
-    return group == 128 && K % 128 == 0 && N % 4 == 0 && gemm_fp8_supported(M, N, K) &&
-           (K / 64) * N * 4 < (1ull << 31);
+    return group == 128 && K % 128 == 0 && gemm_fp8_supported(M, N, K) && (K / 64) * (N + 3) * 4 < (1ull << 31);
 }
 
 bool gemm_fp8_supported(size_t M, size_t N, size_t K) {

@@ -233,8 +233,8 @@ int stage_scales(lx2v_hip_ctx *ctx, lx2v_hip_weight *w) {
 // (load time: one copy to the host and back).
 int group_ratios(lx2v_hip_ctx *ctx, lx2v_hip_weight *w) {
     if (w->fmt != LX2V_WFMT_FP8 || w->group != 128 || w->cols % 128) return LX2V_OK;
-    const size_t rows = w->rows, G = w->cols / 128;
-    std::vector<float> s(rows * G), r(rows * G), last(rows);
+    const size_t rows = w->rows, G = w->cols / 128, stride = gratio_stride(rows);
+    std::vector<float> s(rows * G), r(stride * G, 1.0f), last(rows);
     HIP_TRY(hipMemcpyAsync(s.data(), w->scales, s.size() * 4, hipMemcpyDeviceToHost, ctx->stream), "group scales");
     HIP_TRY(hipStreamSynchronize(ctx->stream), "group scales");
     bool ok = true;
@@ -247,7 +247,7 @@ int group_ratios(lx2v_hip_ctx *ctx, lx2v_hip_weight *w) {
             hi = std::max(hi, sn[g]);
         }
         if (ok && hi > lo * 0x1p60f) ok = false;
-        for (size_t g = 0; g < G; g++) r[g * rows + n] = g == 0 ? 1.0f : sn[g - 1] / sn[g];
+        for (size_t g = 1; g < G; g++) r[g * stride + n] = sn[g - 1] / sn[g];
         last[n] = sn[G - 1];
     }
     w->gratio_ok = ok;

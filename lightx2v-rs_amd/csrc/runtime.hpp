@@ -64,8 +64,9 @@ struct lx2v_hip_weight {
     // the group scales with.  Their accumulator T holds the sum so far in
     // units of the current group's scale, T_g = (s_{g-1} / s_g) T_{g-1} + P_g
     // (P_g the group's raw code products), and the epilogue multiplies by
-    // the last group's scale: gratio [cols / 128][rows] f32 (row g = s_{g-1}
-    // / s_g per channel, row 0 all ones), glast [rows].  gratio_ok: every
+    // the last group's scale: gratio [cols / 128][gratio_stride(rows)] f32 (row
+    // g = s_{g-1} / s_g per channel, row 0 and the padding all ones), glast
+    // [rows].  gratio_ok: every
     // scale finite and > 0 and no channel's scales more than 2^60 apart, so
     // no ratio or partial sum overflows; other grouped weights take the
     // bf16 MFMA kernel (k_gemm_w16) instead.
@@ -77,6 +78,10 @@ struct lx2v_hip_weight {
 };
 
 namespace lx2v {
+
+// Floats per row of lx2v_hip_weight::gratio: the kernels load it 16 bytes a
+// lane, so every row starts on 16 bytes whatever the channel count.
+constexpr size_t gratio_stride(size_t rows) { return (rows + 3) / 4 * 4; }
 
 // Per-kernel timing (Backend::profile_report).
 struct Profiler {

@@ -426,6 +426,62 @@ def test_fp8_g128_mfma_vs_oracle(be, M, K, N):
     assert np.array_equal(u32(y16), u32(O.bf16_round(y)))
 
 
+@pytest.mark.parametrize("M,N", [(1, 33), (129, 130), (257, 1001)])
+@pytest.mark.parametrize("xdt", ["f32", "bf16", "e4m3", "mx"])
+def test_fp8_g128_any_channel_count(be, monkeypatch, xdt, M, N):
+    """Group-128 FP8 with channel counts that are not multiples of 4, on the
+    fp8 MFMA like every other: the few-rows kernel and each grouped tile
+    against the oracle on the quantized activations (per token, or MX), the
+    tiles among each other bit for bit; linear_residual as the pair."""
+    K = 512
+    x, b = O.bf16_round(normal(41 + M, M * K)).reshape(M, K), normal(42, N, 0.01)
+    wf = normal(43 + N, N * K, 0.02).reshape(N, K)
+    wf[:, 128:256] *= np.float32(20.0)  # ratios far from 1, different in every channel
+    q, s = O.fp8_quantize(wf, N, K, 128, True)
+    w, bb = be.weight_fp8(q, s, N, K, 128), be.upload(b)
+    xb = be.alloc(M * K, H.DTYPE_F32 if xdt == "f32" else H.DTYPE_BF16)
+    be.write(xb, x)
+    if xdt in ("e4m3", "mx"):
+        xq = be.alloc_mx(M, K) if xdt == "mx" else be.alloc_e4m3(M, K)
+        (be.quantize_mx if xdt == "mx" else be.quantize_act)(xb, 0, M, xq)
+        xb = xq
+    if xdt == "mx":
+        want = O.linear(O.dequant_mx(*O.act_quant_mx(x)), O.fp8_dequantize(q, s, N, K, 128), b, 1, nthreads=8)
+    else:
+        want = oracle_w8a8(x, q, s, 128, b, 1)
+
+    def run(name, **env):
+        for k in ("ROWS", "FP8_CFG"):
+            monkeypatch.delenv(f"LIGHTX2V_HIP_{k}", raising=False)
+        for k, v in env.items():
+            monkeypatch.setenv(f"LIGHTX2V_HIP_{k}", v)
+        out = []
+        for ydt in (H.DTYPE_F32, H.DTYPE_BF16):
+            y = be.alloc((M + 1) * N, ydt)
+            be.write(y, np.full((M + 1) * N, np.nan, np.float32))
+            _, ks = _kernels(be, lambda: be.linear(xb, 0, M, w, bb, H.ACT_GELU_TANH, y, 0))
+            assert {k for k in ks if k.startswith("gemm")} == {f"gemm_fp8_e4m3.{name}.g128" + (".mxin" if xdt == "mx" else "")}, ks
+            v = be.download(y).reshape(M + 1, N)
+            assert np.isnan(v[M]).all()
+            out.append(v[:M])
+        assert_close(out[0], want, *FP8_TIGHT, what=f"{name} {xdt} {M}x{N}")
+        assert np.array_equal(u32(out[1]), u32(O.bf16_round(out[0]).reshape(M, N)))
+        return out[0]
+
+    if M <= 64:
+        run("rows", ROWS="64")
+    tiles = [run(f"c{c}", FP8_CFG=str(c)) for c in ((0, 1, 10) if xdt == "mx" else (0, 1, 6, 10))]
+    assert all(np.array_equal(u32(tiles[0]), u32(t)) for t in tiles[1:])
+    monkeypatch.delenv("LIGHTX2V_HIP_FP8_CFG")
+    mods, h1, h2, y = be.upload(normal(44, 2 * N)), *(be.alloc(M * N, H.DTYPE_BF16) for _ in range(3))
+    for h in (h1, h2):
+        be.write(h, normal(45, M * N))
+    be.linear_residual(xb, 0, M, w, bb, H.ACT_NONE, h1, 0, mods, 1)
+    be.linear(xb, 0, M, w, bb, H.ACT_NONE, y, 0)
+    be.gate_residual(h2, y, M, N, mods, 1)
+    assert np.array_equal(u32(be.download(h1)), u32(be.download(h2)))
+
+
 def test_fp8_g128_reference_contract(be):
     """The reference's own FP8 weights (its encoder, group 128, exponent-0
     codes included) against the unmodified contract: the oracle's linear
