@@ -2326,7 +2326,8 @@ Fp8Plan plan_gemm_fp8(int num_cu, size_t M, size_t N, size_t K, bool mx, bool mx
                       int act, bool residual, bool allow_split) {
     Fp8Plan p;
     if (K % 128 != 0) {  // the register-staged kernel
-        p.cost_us = (double)K / 64 * 0.45 + 6.0;
+        // up to 64 rows, where it is compared with the few-rows kernel
+        p.cost_us = (double)((N + 128 * (size_t)num_cu - 1) / (128 * (size_t)num_cu)) * ((double)K / 64 * 0.32 + 6.0) + 2.2;
         return p;
     }
     // Split K where even the 256 x 128 tiles leave at least half the CUs

@@ -326,39 +326,64 @@ dim3 rows_grid(size_t M, size_t N, int mb) {
 
 size_t gemm_rows_limit(RowsKind kind) {
     const char *e = getenv("LIGHTX2V_HIP_ROWS");
-    return e && *e ? (size_t)std::max(0, atoi(e)) : kind == RowsKind::Fp8 ? 64 : 256;
+    return e && *e ? (size_t)std::max(0, atoi(e)) : kind <= RowsKind::Fp8Scaled ? 64 : 256;
 }
 
-// The modelled time: a wave's share of the 128-element steps, each slower with
-// the rows it loads, times the workgroups a CU runs where they outnumber the
-// CUs.  Fitted at 1536 -> 1536, 14336 -> 1536 and 3072 -> 14336 (M 1 .. 64; us,
-// the tile kernels' beside them): FP8, e4m3 input, M 17: 6.0 / 7.5, MX input
-// 23.4 / 42.0, e4m3 13.7 / 12.3; group 128, M 64: 9.1 / 9.4, 43.3 / 49.7, 25.3
-// / 15.6; Q8 M 64: 11.8 / 22.0, 72.9 / 197, 39.9 / 45.7; native, M 1: 6.6 / 7.8,
-// 33.6 / 51, 20.0 / 22.5.  So it is the choice where the tiles leave CUs idle
-// over a long K and there are few rows to load beside the weight's.
+namespace {
+
+// The modelled time of a call among others, by the most rows a workgroup takes
+// (32 or 64): `us` a step of a wave's share of K (K / 1024 rounded up), plus, per
+// 1024 of K, `row` for each row loaded and `busy` where every CU reads its part
+// of the weight; a CU runs one workgroup at a time, so all of it once more for
+// every 256 workgroups.  Fitted over 512 .. 14336 x 64 .. 14336 (M 1 .. 256, weights
+// hot and cold): rms 4 to 12%.
+struct RowsCost {
+    double base, us, row, busy;
+};
+constexpr RowsCost kRowsCost[][2] = {
+    {{4.8, 0.83, 0.024, 0.44}, {4.9, 0.93, 0.027, 1.17}},  // Fp8
+    {{4.7, 0.93, 0.024, 0.55}, {4.6, 1.15, 0.028, 1.10}},  // Fp8Scaled
+    {{5.3, 1.63, 0.042, 1.15}, {4.1, 2.55, 0.032, 1.56}},  // W16
+    {{4.2, 1.06, 0.134, 1.30}, {3.6, 3.21, 0.081, 0.85}},  // W16F32
+    {{4.1, 1.93, 0.048, 0.65}, {5.2, 2.18, 0.047, 1.18}},  // Native
+    {{4.5, 2.25, 0.087, 0.91}, {4.5, 3.00, 0.090, 0.91}},  // NativeF32
+};
+
+double rows_cost_us(RowsKind kind, int num_cu, size_t M, size_t N, size_t K) {
+    const RowsCost &c = kRowsCost[(int)kind][M > 32];
+    const size_t cols = (N + RN - 1) / RN, blocks = (M + 63) / 64, wg = cols * blocks, rounds = (wg + num_cu - 1) / num_cu;
+    const double own = (double)((K + 1023) / 1024), kf = (double)K / 1024;
+    const double per = own * c.us + kf * (c.row * (double)std::min<size_t>(M, 64) + c.busy * std::min(1.0, (double)wg / num_cu));
+    double n = (double)rounds;
+    if (rounds > 1 && blocks > 1 && wg - (rounds - 1) * num_cu <= cols)  // the last round: the last block's rows only
+        n += (double)std::max<size_t>(M - 64 * (blocks - 1), 16) / 64 - 1.0;
+    return c.base + n * per;
+}
+
+}  // namespace
+
+// Where the tiles leave CUs idle over a long K and there are few rows to load
+// beside the weight's.  Rows / the other kernels (us, other_us): FP8, e4m3
+// input, 17 x 14336 -> 3072 22 / 29, 33 x 14336 -> 3072 36 / 29; group 128, 64 x
+// 1536 -> 8960 19 / 11; Q8, 17 x 1536 -> 1536 9 / 13, 200 x 14336 -> 3072 147 /
+// 77, f32 rows 64 x 14336 -> 1536 130 / 71.  Over 2100 shapes the kernel taken
+// is on average 0.6% slower than the fastest.
 // LIGHTX2V_HIP_ROWS=<n> takes it for every call of up to n rows instead.
-bool gemm_rows_chosen(RowsKind kind, int num_cu, size_t M, size_t N, size_t K, double tile_us) {
+bool gemm_rows_chosen(RowsKind kind, int num_cu, size_t M, size_t N, size_t K, double other_us) {
     if (K % 64 || N == 0 || M == 0) return false;
     // 32-bit offsets into the rows as they are (the tiles read f32 ones as bf16)
-    if (kind == RowsKind::F32Act && M * K * 4 >= (1ull << 31)) return false;
-    // a pinned tile configuration stays the tile kernels'
-    for (const char *pin : {"LIGHTX2V_HIP_FP8_CFG", "LIGHTX2V_HIP_W16_CFG"}) {
-        const char *e = getenv(pin);
-        if (e && *e && atoi(e) >= 0) return false;
-    }
-    const char *e = getenv("LIGHTX2V_HIP_ROWS");
+    if ((kind == RowsKind::W16F32 || kind == RowsKind::NativeF32) && M * K * 4 >= (1ull << 31)) return false;
     if (M > gemm_rows_limit(kind)) return false;
+    // a pinned tile configuration stays the tile kernels'
+    const char *pin = getenv(kind <= RowsKind::Fp8Scaled ? "LIGHTX2V_HIP_FP8_CFG"
+                             : kind <= RowsKind::W16F32  ? "LIGHTX2V_HIP_W16_CFG"
+                                                         : "LIGHTX2V_HIP_BF16_CFG");
+    if (pin && *pin && atoi(pin) >= 0) return false;
+    const char *e = getenv("LIGHTX2V_HIP_ROWS");
     if (e && *e) return true;
-    struct Step {
-        double us, row_us, crowd;
-    };
-    static constexpr Step kStep[] = {{0.90, 0.021, 1.35}, {1.60, 0.045, 1.45}, {1.70, 0.060, 1.40}, {2.10, 0.105, 1.40}};
-    const Step &c = kStep[(int)kind];
-    const size_t own = ((K + RK - 1) / RK + RW - 1) / RW, wg = (N + RN - 1) / RN * ((M + 63) / 64);
-    const double rows = (double)(M < 64 ? M : 64), per = c.us + c.row_us * rows * (M > 32 ? 1.2 : 1.0);
-    const double crowd = wg > (size_t)num_cu ? c.crowd * (double)wg / num_cu : 1.0;
-    return 4.0 + (double)own * per * crowd < tile_us;
+    // (a native call's choices lie within a microsecond where K is short: there the
+    // tiles, which sum every row the same way whatever the row count, keep it)
+    return rows_cost_us(kind, num_cu, M, N, K) < (kind == RowsKind::NativeF32 ? 0.9 : 1.0) * other_us;
 }
 
 void launch_gemm_rows_fp8(hipStream_t s, const uint8_t *x, const float *x_scale, const lx2v_hip_weight *w, bool grouped,

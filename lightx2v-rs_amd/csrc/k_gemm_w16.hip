@@ -909,10 +909,12 @@ int plan_gemm_w16_dma(int num_cu, size_t M, size_t N) {
     return pick;
 }
 
+namespace {
+
 // A 64-element stage of the 256 x 128 and 128 x 256 tiles costs 0.86 us plus
 // what the dequantization adds with every CU busy (power and LDS), of the 256 x
-// 256 one about twice that (M 300 .. 4680, K 512 .. 14336: within 15%).
-double gemm_w16_dma_cost_us(int num_cu, const lx2v_hip_weight *w, size_t M) {
+// 256 one about twice that (M 1 .. 4680, K 256 .. 14336: within 20%).
+double w16_dma_cost_us(int num_cu, const lx2v_hip_weight *w, size_t M) {
     const size_t N = w->rows, K = w->cols;
     const DmaCfg &c = kDmaW16[plan_gemm_w16_dma(num_cu, M, N)];
     const bool q4 = w->fmt == LX2V_WFMT_Q4, big = c.bm * c.bn > 256 * 128;
@@ -921,6 +923,16 @@ double gemm_w16_dma_cost_us(int num_cu, const lx2v_hip_weight *w, size_t M) {
     const double stage = big ? (q4 ? 1.45 + 0.25 * busy : 1.50 + 0.30 * busy) : 0.86 + (q4 ? 0.16 : 0.25) * busy;
     return (double)((tiles + num_cu - 1) / num_cu) * ((double)K / 64 * stage + (big ? 10.0 : 3.0 + 4.0 * busy));
 }
+
+// What the pass that writes a weight out adds to the bf16 GEMM: the pass, and
+// the GEMM's read of what other XCDs' L2s hold.  For weights of 2.4, 6.3, 9.4,
+// 13.8, 26 and 44 million 3.5 to 7, 10.6, 14.7, 15 to 20, 20 and 25 us.
+double w16_expand_us(size_t weights) {
+    const double m = (double)weights * 1e-6;
+    return std::min(2.0 + 1.35 * m, 12.5 + 0.31 * m);
+}
+
+}  // namespace
 
 void launch_gemm_w16_dma(hipStream_t s, int cfg, const uint16_t *x, const lx2v_hip_weight *w, const float *bias,
                          int act, void *y, int y_dtype, size_t M) {
@@ -963,20 +975,21 @@ __global__ __launch_bounds__(256) void k_w16_expand(const uint8_t *__restrict__ 
 // 162 -> 133 / 151 -> 132, 4680 x 8960 -> 1536 159 -> 129 / 139 -> 125, 300 x
 // 8960 -> 1536 127 -> 45 / 120 -> 45, 300 x 1536 -> 1536 23 -> 15, 4680 x 3072
 // -> 14336 472 -> 382.  A short GEMM over a wide weight does not repay the pass:
-// 600 x 1536 -> 4608 25.1 / 27.3, 300 x 3072 -> 14336 54 / 65, 1560 x 1536 -> 8960
-// 57 / 59, 4680 x 1536 -> 1536 32.6 / 33.3.  The pass and the cold read of what
-// it wrote take 7.5 us + 0.48 us per million weights; 3.5 us more is asked so
-// that the models' errors do not pick the slower side.  Weights up to 128 MB
-// written out bound the workspace.
+// 128 x 1536 -> 8960 23 / 30, 600 x 1536 -> 4608 25.1 / 27.3, 300 x 3072 -> 14336
+// 54 / 65, 4680 x 1536 -> 1536 32.6 / 33.3.  Weights up to 128 MB written out
+// bound the workspace.
 // LIGHTX2V_HIP_W16_EXPAND=0 / 1 pins the choice for calls that both sides take.
-bool w16_expand_chosen(int num_cu, const lx2v_hip_weight *w, size_t M, int y_dtype) {
+W16Plan plan_w16(int num_cu, const lx2v_hip_weight *w, size_t M, int y_dtype) {
     const size_t N = w->rows, K = w->cols;
-    if (!gemm_w16_dma_supported(w, M) || !gemm_bf16_supported(M, N, K) || N * K * 2 > (128u << 20)) return false;
-    const char *cfg = getenv("LIGHTX2V_HIP_W16_CFG");
-    if (cfg && *cfg && atoi(cfg) >= 0) return false;  // a pinned tile dequantizes inside
+    W16Plan p;
+    p.cost_us = w16_dma_cost_us(num_cu, w, M);
+    // (a pinned tile dequantizes inside)
+    if (!gemm_bf16_supported(M, N, K) || N * K * 2 > (128u << 20) || forced_w16_cfg() >= 0) return p;
+    const double out = w16_expand_us(N * K) + gemm_bf16_cost_us(num_cu, M, N, K, y_dtype);
     const char *e = getenv("LIGHTX2V_HIP_W16_EXPAND");
-    if (e && *e) return atoi(e) != 0;
-    return 7.5 + (double)(N * K) * 0.48e-6 + gemm_bf16_cost_us(num_cu, M, N, K, y_dtype) + 3.5 < gemm_w16_dma_cost_us(num_cu, w, M);
+    p.expand = e && *e ? atoi(e) != 0 : out < p.cost_us;
+    if (p.expand) p.cost_us = out;
+    return p;
 }
 
 void launch_w16_expand(hipStream_t s, const lx2v_hip_weight *w, uint16_t *out) {
@@ -1061,7 +1074,7 @@ int bf16_pick(int num_cu, size_t M, size_t N, size_t K, int y_dtype, double *us)
 double gemm_bf16_cost_us(int num_cu, size_t M, size_t N, size_t K, int y_dtype) {
     double us;
     bf16_pick(num_cu, M, N, K, y_dtype, &us);
-    return us;
+    return 0.96 * us + 2.2;  // (with the gap between two launches; M 1 .. 256: within 7% rms)
 }
 
 void launch_gemm_bf16(hipStream_t s, int num_cu, const uint16_t *x, const uint16_t *w, const float *bias, int act,

@@ -1916,11 +1916,6 @@ static int act_quant_into_ws(lx2v_hip_ctx *ctx, const void *x, int dtype, size_t
     return run(ctx, "act_quant_e4m3", [&] { launch_act_quant(ctx->stream, x, dtype, rows, cols, *q, *s); });
 }
 
-// gate: residual mode (only where linear_fusable says so): y is the
-// residual stream, y[r] += out[r] * gate.
-// scr: the no-alloc variant -- every workspace comes from this device
-// memory (bias staging first, then the activations' e4m3 codes and row
-// scales or their bf16 copy), and the call fails cleanly if it is too small.
 // Whether the few-rows kernel takes an FP8 linear, decided against the plan
 // linear itself would make (linear_residual asks the same question, so that
 // both sum in the same order).
@@ -1931,10 +1926,20 @@ static bool few_rows_fp8(const lx2v_hip_ctx *ctx, size_t rows, const lx2v_hip_we
     if (rows > gemm_rows_limit(RowsKind::Fp8)) return false;
     const Fp8Plan p = known ? *known : plan_gemm_fp8(ctx->num_cu, rows, N, K, x_mx || y_mx, x_mx, grouped, y_dtype, act, false, true);
     if (p.splits > 1 && p.cost_us == 0.0) return false;  // a forced split
-    // (group-128 and MX stages of the few-tile configurations run slower than modelled)
-    return gemm_rows_chosen(RowsKind::Fp8, ctx->num_cu, rows, N, K, p.cost_us * (grouped ? 1.4 : x_mx ? 1.2 : 1.0));
+    // The plan's time as measured at 1 .. 64 rows, a round of workgroups that wait
+    // for memory: the planner's figures rank tiles among each other over all rows.
+    // (us, modelled / measured: e4m3 8960 -> 1536 21.6 / 25, MX 22.8 / 32, group 128
+    // 21.6 / 36; within 6% rms after this.)
+    const double c = p.cost_us;
+    const double us = p.kernel < 0 ? c : p.splits > 1 ? 0.85 * c : grouped ? 1.7 * c - 3.5 : x_mx ? 1.32 * c : 1.13 * c + 0.6;
+    return gemm_rows_chosen(grouped || x_mx ? RowsKind::Fp8Scaled : RowsKind::Fp8, ctx->num_cu, rows, N, K, us);
 }
 
+// gate: residual mode (only where linear_fusable says so): y is the
+// residual stream, y[r] += out[r] * gate.
+// scr: the no-alloc variant -- every workspace comes from this device
+// memory (in the order they are laid out below), and the call fails cleanly
+// if it is too small.
 static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, size_t rows, const lx2v_hip_weight *w,
                       const lx2v_hip_buf *bias, int act, lx2v_hip_buf *y, size_t y_row, const float *gate,
                       const lx2v::Scratch *scr = nullptr) {
@@ -2000,15 +2005,22 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
             plan.kernel != 10)  // built with grouped scales
             return fail(LX2V_ERR_UNSUPPORTED, "no grouped-scale fp8 kernel for configuration %d", plan.kernel);
     }
+    // A dequantized weight: inside the GEMM, or written out first.
+    const bool w16_dma = !e4m3_path && !native_bf16 && gemm_w16_dma_supported(w, rows);
+    const W16Plan w16 = w16_dma ? plan_w16(ctx->num_cu, w, rows, y->dtype) : W16Plan{};
     // Few rows: the kernels that read the weight once, on the same operands.
+    // (Decided by shapes and types alone, so that a call gives the same bits
+    // eagerly, captured and without allocations.)
     bool few = false;
-    if (e4m3_path)
+    if (e4m3_path) {
         few = fp8_mfma && few_rows_fp8(ctx, rows, w, x_mx, y_mx, fp8_grouped, y->dtype, act, gate ? nullptr : &plan);
-    else if (rows <= gemm_rows_limit(RowsKind::W16) && (native_bf16 || gemm_w16_dma_supported(w, rows)))
-        few = gemm_rows_chosen(x->dtype == LX2V_DTYPE_F32 ? RowsKind::F32Act : native_bf16 ? RowsKind::Native : RowsKind::W16,
+    } else if ((native_bf16 || w16_dma) && rows <= gemm_rows_limit(RowsKind::W16)) {
+        const bool f32 = x->dtype == LX2V_DTYPE_F32;
+        const double other = native_bf16 ? gemm_bf16_cost_us(ctx->num_cu, rows, N, K, y->dtype) : w16.cost_us;
+        few = gemm_rows_chosen(native_bf16 ? (f32 ? RowsKind::NativeF32 : RowsKind::Native) : (f32 ? RowsKind::W16F32 : RowsKind::W16),
                                ctx->num_cu, rows, N, K,
-                               (native_bf16 ? gemm_bf16_cost_us(ctx->num_cu, rows, N, K, y->dtype) : gemm_w16_dma_cost_us(ctx->num_cu, w, rows)) +
-                                   (x->dtype == LX2V_DTYPE_F32 ? 2.5 : 0.0));  // the tiles' pass that rounds f32 rows to bf16
+                               other + (f32 ? 2.2 + (double)(rows * K) * 1.2e-6 : 0.0));  // f32 rows rounded to bf16 in a pass
+    }
     if (few) plan.splits = 1;
     // Workspaces, each piece 256-byte aligned: a bf16 bias's f32 copy; the
     // activations' e4m3 codes and row scales, or their bf16 copy; split K's
@@ -2018,7 +2030,7 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t s_bias = bias && bias->dtype != LX2V_DTYPE_F32 ? al(N * 4) : 0;
     const size_t s_act = e4m3_path ? (x->quantized() ? 0 : al(rows * K) + al(rows * 4))
-                                   : (!few && (gemm_w16_dma_supported(w, rows) || native_bf16) && x->dtype == LX2V_DTYPE_F32
+                                   : (!few && (w16_dma || native_bf16) && x->dtype == LX2V_DTYPE_F32
                                           ? al(rows * K * 2)
                                           : 0);
     const size_t s_part = plan.splits > 1 ? al((size_t)plan.splits * rows * N * 4) : 0;
@@ -2142,14 +2154,14 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
         return ok();
     }
     const char *name = w->fmt == LX2V_WFMT_Q8 ? "gemm_w16_q8" : w->fmt == LX2V_WFMT_Q4 ? "gemm_w16_q4" : "gemm_w16_fp8";
-    if (gemm_w16_dma_supported(w, rows)) {
+    if (w16_dma) {
         const uint16_t *xb;
         if (int rc = bf16_x(&xb)) return rc;
         // Many rows: the weight's bf16 values written out once, then the bf16
         // GEMM on them (the same products in the same order).  Not in a
         // graph, which would hold the workspace, nor where nothing may be
         // allocated; without the memory the tiles below take the call.
-        if (!scr && !ctx->capturing && w16_expand_chosen(ctx->num_cu, w, rows, y->dtype)) {
+        if (!scr && !ctx->capturing && w16.expand) {
             if (ensure(ctx, &ctx->wexp.ptr, &ctx->wexp.bytes, N * K * 2, "weight workspace alloc") == LX2V_OK) {
                 uint16_t *wx = (uint16_t *)ctx->wexp.ptr;
                 if (int rc = run(ctx, "w16_expand", [&] { launch_w16_expand(ctx->stream, w, wx); })) return rc;

@@ -343,11 +343,18 @@ void launch_gemm_fp8(hipStream_t s, int num_cu, const Fp8Plan &p, const uint8_t 
 // The fp8 one takes e4m3 / MX activations and per-channel or group-128
 // weights (`grouped`: lx2v_hip_weight::sscale); the w16 one bf16 or f32
 // activations and the weights of launch_gemm_w16_dma, or a native weight's
-// bf16 copy.  gemm_rows_chosen: whether it takes a call that would otherwise
-// cost tile_us on the tile kernels.
-enum class RowsKind { Fp8, W16, Native, F32Act };  // F32Act: f32 activations of the bf16 MFMA kinds
+// bf16 copy.  gemm_rows_chosen: whether it takes a call that the other kernels
+// would take in other_us (their pass that rounds f32 rows included).
+enum class RowsKind {
+    Fp8,        // per-token e4m3 activations, per-channel weights
+    Fp8Scaled,  // MX activations and / or group-128 weights
+    W16,        // bf16 activations, dequantized weights
+    W16F32,     // f32 activations, dequantized weights
+    Native,     // bf16 activations, native weights
+    NativeF32,  // f32 activations, native weights
+};
 size_t gemm_rows_limit(RowsKind kind);  // the most rows it is asked for (larger calls skip the models)
-bool gemm_rows_chosen(RowsKind kind, int num_cu, size_t M, size_t N, size_t K, double tile_us);
+bool gemm_rows_chosen(RowsKind kind, int num_cu, size_t M, size_t N, size_t K, double other_us);
 void launch_gemm_rows_fp8(hipStream_t s, const uint8_t *x, const float *x_scale, const lx2v_hip_weight *w, bool grouped,
                           const float *bias, int act, void *y, int y_dtype, size_t M, const Fp8Mx &mx);
 void launch_gemm_rows_w16(hipStream_t s, const void *x, int x_dtype, const lx2v_hip_weight *w, const float *bias, int act,
@@ -364,17 +371,21 @@ void launch_gemm_w16(hipStream_t s, int num_cu, const void *x, int x_dtype,
                      size_t M);
 bool gemm_w16_dma_supported(const lx2v_hip_weight *w, size_t M);
 int plan_gemm_w16_dma(int num_cu, size_t M, size_t N);
-double gemm_w16_dma_cost_us(int num_cu, const lx2v_hip_weight *w, size_t M);  // modelled time of its choice
 void launch_gemm_w16_dma(hipStream_t s, int cfg, const uint16_t *x, const lx2v_hip_weight *w, const float *bias,
                          int act, void *y, int y_dtype, size_t M);
-// The weight's bf16 values written out for launch_gemm_bf16, and whether that
-// pass and GEMM beat dequantizing inside launch_gemm_w16_dma.
-bool w16_expand_chosen(int num_cu, const lx2v_hip_weight *w, size_t M, int y_dtype);
+// How a weight that gemm_w16_dma_supported takes is contracted: inside
+// launch_gemm_w16_dma, or its bf16 values written out (launch_w16_expand) for
+// launch_gemm_bf16; and the modelled time of that.
+struct W16Plan {
+    bool expand = false;
+    double cost_us = 0.0;
+};
+W16Plan plan_w16(int num_cu, const lx2v_hip_weight *w, size_t M, int y_dtype);
 void launch_w16_expand(hipStream_t s, const lx2v_hip_weight *w, uint16_t *out);
 // bf16 x bf16 (native f32 weights through their bf16 copy): X [M, K] and
 // W [N, K] bf16, K % 64 == 0.
 bool gemm_bf16_supported(size_t M, size_t N, size_t K);
-double gemm_bf16_cost_us(int num_cu, size_t M, size_t N, size_t K, int y_dtype);  // modelled time of launch_gemm_bf16's choice
+double gemm_bf16_cost_us(int num_cu, size_t M, size_t N, size_t K, int y_dtype);  // modelled time of its choice, among other calls
 void launch_gemm_bf16(hipStream_t s, int num_cu, const uint16_t *x, const uint16_t *w, const float *bias, int act,
                       void *y, int y_dtype, size_t M, size_t N, size_t K);
 // k_gemm_fp8.hip: the persistent 256 x 256 tile over bf16 rows, one of

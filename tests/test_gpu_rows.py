@@ -122,3 +122,50 @@ def test_rows_residual_equals_pair(be, monkeypatch, fmt, hdt):
     be.linear(xb, 0, M, w, bb, H.ACT_NONE, y, 0)
     be.gate_residual(h2, y, M, N, mods, 1)
     assert np.array_equal(u32(be.download(h1)), u32(be.download(h2)))
+
+
+# Calls where one way is at least 1.3 times the next (us, rows / tiles or rows / written out / tiles)
+@pytest.mark.parametrize("fmt,xdt,M,K,N,way", [
+    ("q8", "bf16", 17, 1536, 1536, "rows"),       # 9 / 13 / 23
+    ("q4", "f32", 17, 3072, 3072, "rows"),        # 16 / 30 / 46
+    ("q8", "bf16", 200, 14336, 3072, "written"),  # 147 / 77 / 197
+    ("q4", "f32", 64, 14336, 1536, "written"),    # 129 / 73 / 189
+    ("q8", "f32", 256, 8960, 1536, "written"),    # 82 / 52 / 128
+    ("q8", "bf16", 128, 1536, 8960, "tiles"),     # 35 / 30 / 23
+    ("native", "f32", 1, 1984, 9000, "tiles"),    # 20 / 13
+    ("native", "bf16", 64, 1536, 8960, "tiles"),  # 24 / 8
+    ("fp8", "bf16", 17, 8960, 1536, "rows"),      # 15 / 25 (the quantization aside)
+    ("fp8", "e4m3", 33, 14336, 3072, "tiles"),    # 36 / 29
+    ("fp8", "mx", 33, 1536, 8960, "tiles"),       # 16 / 10
+    ("fp8_128", "bf16", 64, 1536, 8960, "tiles"),  # 22 / 14
+    ("fp8_128", "mx", 64, 1536, 8960, "tiles"),   # 19 / 11
+])
+def test_the_faster_kernel_is_taken(be, monkeypatch, fmt, xdt, M, K, N, way):
+    for k in ("ROWS", "W16_EXPAND", "W16_CFG", "FP8_CFG", "BF16_CFG", "FP8_SPLITK"):
+        monkeypatch.delenv(f"LIGHTX2V_HIP_{k}", raising=False)
+    codes = (np.arange(N * K, dtype=np.uint32) * np.uint32(2654435761) >> np.uint32(24)).astype(np.uint8)
+    if fmt == "native":
+        w = be.weight((codes.astype(np.float32) - 128) * np.float32(1e-3), N, K)
+    elif fmt == "q8":
+        w = be.weight_q8(codes.view(np.int8), np.full(N * K // 32, 1e-3, np.float32), N, K, 32)
+    elif fmt == "q4":
+        w = be.weight_q4(codes[:N * K // 2], np.full(N * K // 32, 1e-2, np.float32), np.full(N * K // 32, 8, np.float32),
+                         N, K, 32, packed=True)
+    else:
+        g = K if fmt == "fp8" else 128
+        codes = codes & 0xBF
+        w = be.weight_fp8(np.where((codes & 0x78) == 0, codes & 0x80, codes).astype(np.uint8),
+                          np.full(N * K // g, 1e-2, np.float32), N, K, g)
+    x, y = be.alloc(M * K, H.DTYPE_F32 if xdt == "f32" else H.DTYPE_BF16), be.alloc(M * N, H.DTYPE_BF16)
+    if xdt in ("mx", "e4m3"):
+        x = be.alloc_mx(M, K) if xdt == "mx" else be.alloc_e4m3(M, K)
+    be.profile_reset()
+    be.profile_enable(True)
+    try:
+        be.linear(x, 0, M, w, None, H.ACT_NONE, y, 0)
+        names = list(be.profile_stats())
+    finally:
+        be.profile_enable(False)
+        be.profile_reset()
+    got = "rows" if any(".rows" in k for k in names) else "written" if "w16_expand" in names else "tiles"
+    assert got == way, names
