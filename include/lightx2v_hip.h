@@ -444,12 +444,15 @@ int lx2v_hip_linear(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, size
 
 /* No counterpart in the reference: lx2v_hip_linear for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses
- * that forbid hipMalloc).  Same arguments, plan, kernels and results as
+ * that forbid hipMalloc).  Same arguments, plan and results as
  * lx2v_hip_linear, bit for bit; its workspaces (the per-token e4m3
  * activations and row scales, a bf16 bias's f32 copy, f32 activations' bf16
- * copy, split K's f32 partial sums) live in a device array of 48 MiB per
- * device instead of the context's, so it calls no hipMalloc / hipFree and
- * records no profiler events.  A call needing more (roughly rows * cols >
+ * copy, split K's f32 partial sums, a Q8 / Q4 / FP8-group weight written out
+ * as bf16) live in a device array of 48 MiB per device instead of the
+ * context's, so it calls no hipMalloc / hipFree and records no profiler
+ * events.  Where a weight written out does not fit beside the rest, the GEMM
+ * dequantizes it inside: other kernels, the same bits.  A call needing more
+ * than the array for the others (roughly rows * cols >
  * 48 MiB with f32 / bf16 activations, plus S * rows * w.rows * 4 bytes where
  * K is split S ways) fails with LX2V_ERR_UNSUPPORTED and a message and
  * enqueues nothing; pre-quantized E4M3 / MXE4M3 activations need no
@@ -475,7 +478,11 @@ int lx2v_hip_act_quant(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, s
  * context stream once and replay it with one launch.  Between begin and end
  * only those calls are allowed (anything that allocates, frees, transfers
  * host memory or synchronises fails with LX2V_ERR_UNSUPPORTED); run the
- * sequence once eagerly first so workspaces are already large enough.
+ * sequence once eagerly first so workspaces are already large enough.  (The
+ * one that is not needed is a Q8 / Q4 / FP8-group weight's bf16 values: without
+ * room for them the GEMM dequantizes inside, slower, with the same bits.)
+ * Workspaces that later calls outgrow stay allocated until the context's last
+ * graph is freed.
  * Replays read and write the buffers captured, at their current contents. */
 typedef struct lx2v_hip_graph lx2v_hip_graph;
 int lx2v_hip_graph_begin(lx2v_hip_ctx *ctx);

@@ -51,14 +51,25 @@ int ok() {
 
 bool valid_dtype(int d) { return d == LX2V_DTYPE_F32 || d == LX2V_DTYPE_BF16; }
 
+// A workspace block that is outgrown: freed, or kept for the captured graphs
+// that may hold its address (until the last one is freed).
+int release(lx2v_hip_ctx *ctx, void *ptr, const char *what) {
+    if (ctx->graphs) {
+        ctx->outgrown.push_back(ptr);
+        return LX2V_OK;
+    }
+    HIP_TRY(hipStreamSynchronize(ctx->stream), what);
+    HIP_TRY(hipFree(ptr), what);
+    return LX2V_OK;
+}
+
 int ensure(lx2v_hip_ctx *ctx, void **ptr, size_t *have, size_t need, const char *what) {
     if (*have >= need) return LX2V_OK;
     if (ctx->capturing)
         return fail(LX2V_ERR_UNSUPPORTED, "%s: would grow a workspace during graph capture (run the sequence "
                     "once before capturing)", what);
     if (*ptr) {
-        HIP_TRY(hipStreamSynchronize(ctx->stream), what);
-        HIP_TRY(hipFree(*ptr), what);
+        if (int rc = release(ctx, *ptr, what)) return rc;
         *ptr = nullptr;
         *have = 0;
     }
@@ -68,6 +79,27 @@ int ensure(lx2v_hip_ctx *ctx, void **ptr, size_t *have, size_t need, const char 
     return LX2V_OK;
 }
 
+// Room for a weight written out (lx2v_hip_ctx::wexp), or false: another path
+// takes the call.  The new block is allocated before the old one goes, and a
+// size the device had no room for is not asked for again until this context
+// frees something.
+bool expand_room(lx2v_hip_ctx *ctx, size_t need) {
+    if (ctx->wexp.bytes >= need) return true;
+    if (ctx->capturing || need >= ctx->wexp_refused) return false;
+    void *p = nullptr;
+    if (hipMalloc(&p, need) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->wexp_refused = need;
+        return false;
+    }
+    if (ctx->wexp.ptr && release(ctx, ctx->wexp.ptr, "weight workspace") != LX2V_OK) {
+        (void)hipFree(p);
+        return false;
+    }
+    ctx->wexp.ptr = p;
+    ctx->wexp.bytes = need;
+    return true;
+}
 
 // Byte ranges [a, a+na) and [b, b+nb) overlap.
 bool overlap(const void *a, size_t na, const void *b, size_t nb) {
@@ -339,6 +371,7 @@ int lx2v_hip_destroy(lx2v_hip_ctx *ctx) {
     if (ctx->ws) (void)hipFree(ctx->ws);
     for (lx2v::Stage *x : {&ctx->stage, &ctx->mask, &ctx->kv_spare, &ctx->resid, &ctx->attn, &ctx->wexp, &ctx->splitk})
         if (x->ptr) (void)hipFree(x->ptr);
+    for (void *p : ctx->outgrown) (void)hipFree(p);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return ok();
@@ -513,6 +546,7 @@ int lx2v_hip_buf_free(lx2v_hip_ctx *ctx, lx2v_hip_buf *buf) {
     if (int rc = set_dev(ctx)) return rc;
     HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize(free)");
     (void)hipFree(buf->ptr);
+    ctx->wexp_refused = SIZE_MAX;
     delete buf;
     return ok();
 }
@@ -688,6 +722,7 @@ int lx2v_hip_weight_free(lx2v_hip_ctx *ctx, lx2v_hip_weight *w) {
     if (int rc = set_dev(ctx)) return rc;
     HIP_TRY(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize(weight_free)");
     free_weight(w);
+    ctx->wexp_refused = SIZE_MAX;
     return ok();
 }
 
@@ -1428,6 +1463,7 @@ int lx2v_hip_kv_cache_free(lx2v_hip_ctx *ctx, lx2v_hip_kv *kv) {
     if (kv->plan_host) (void)hipHostFree(kv->plan_host);
     (void)hipEventDestroy(kv->plan_done);
     delete kv;
+    ctx->wexp_refused = SIZE_MAX;
     return ok();
 }
 
@@ -1864,6 +1900,7 @@ int lx2v_hip_graph_end(lx2v_hip_ctx *ctx, lx2v_hip_graph **out) {
         delete gr;
         return hip_fail(e, "hipGraphInstantiate");
     }
+    ctx->graphs++;
     *out = gr;
     return ok();
 }
@@ -1902,6 +1939,10 @@ int lx2v_hip_graph_free(lx2v_hip_ctx *ctx, lx2v_hip_graph *g) {
     if (g->exec) (void)hipGraphExecDestroy(g->exec);
     if (g->graph) (void)hipGraphDestroy(g->graph);
     delete g;
+    if (--ctx->graphs == 0) {
+        for (void *p : ctx->outgrown) (void)hipFree(p);
+        ctx->outgrown.clear();
+    }
     return ok();
 }
 
@@ -2024,9 +2065,12 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
     if (few) plan.splits = 1;
     // Workspaces, each piece 256-byte aligned: a bf16 bias's f32 copy; the
     // activations' e4m3 codes and row scales, or their bf16 copy; split K's
-    // f32 partial sums.  The no-alloc variant lays them out in that order in
-    // the device scratch; `linear` keeps them in context workspaces, all
-    // grown here, before the first launch.
+    // f32 partial sums; a weight written out as bf16.  The no-alloc variant
+    // lays them out in that order in the device scratch; `linear` keeps them
+    // in context workspaces, all grown here, before the first launch.  Where
+    // there is no room for the written-out weight (p_exp stays null: past the
+    // scratch, a workspace that a capture may not grow, no memory) the tiles
+    // dequantize inside the GEMM, bit for bit the same.
     auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t s_bias = bias && bias->dtype != LX2V_DTYPE_F32 ? al(N * 4) : 0;
     const size_t s_act = e4m3_path ? (x->quantized() ? 0 : al(rows * K) + al(rows * 4))
@@ -2042,10 +2086,14 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
     if (int rc = set_dev(ctx)) return rc;
     uint8_t *p_bias = nullptr, *p_act = nullptr;
     float *p_part = nullptr;
+    uint16_t *p_exp = nullptr;
+    const size_t s_exp = !few && w16.expand ? al(N * K * 2) : 0;
     if (scr) {
         p_bias = scr->ptr;
         p_act = scr->ptr + s_bias;
         p_part = (float *)(scr->ptr + s_bias + s_act);
+        if (s_exp && s_bias + s_act + s_part + s_exp <= scr->bytes)
+            p_exp = (uint16_t *)(scr->ptr + s_bias + s_act + s_part);
     } else {
         void *st = nullptr;
         if (s_bias)  // slot 0 of the staging (linear_residual's gate is in slot 2)
@@ -2055,6 +2103,7 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
         if (s_part)
             if (int rc = ensure(ctx, &ctx->splitk.ptr, &ctx->splitk.bytes, s_part, "split-K workspace alloc"))
                 return rc;
+        if (s_exp && expand_room(ctx, s_exp)) p_exp = (uint16_t *)ctx->wexp.ptr;
         p_bias = (uint8_t *)st;
         p_act = (uint8_t *)ctx->ws;
         p_part = (float *)ctx->splitk.ptr;
@@ -2157,23 +2206,15 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
     if (w16_dma) {
         const uint16_t *xb;
         if (int rc = bf16_x(&xb)) return rc;
-        // Many rows: the weight's bf16 values written out once, then the bf16
-        // GEMM on them (the same products in the same order).  Not in a
-        // graph, which would hold the workspace, nor where nothing may be
-        // allocated; without the memory the tiles below take the call.
-        if (!scr && !ctx->capturing && w16.expand) {
-            if (ensure(ctx, &ctx->wexp.ptr, &ctx->wexp.bytes, N * K * 2, "weight workspace alloc") == LX2V_OK) {
-                uint16_t *wx = (uint16_t *)ctx->wexp.ptr;
-                if (int rc = run(ctx, "w16_expand", [&] { launch_w16_expand(ctx->stream, w, wx); })) return rc;
-                char xname[40];
-                snprintf(xname, sizeof xname, "%s.bf16", name);
-                if (int rc = run(ctx, xname, [&] {
-                        launch_gemm_bf16(ctx->stream, ctx->num_cu, xb, wx, bp, act, yp, y->dtype, rows, N, K);
-                    }))
-                    return rc;
-                return ok();
-            }
-            (void)hipGetLastError();
+        if (p_exp) {  // the weight's bf16 values written out once, then the bf16 GEMM: the same products in the same order
+            if (int rc = run(ctx, "w16_expand", [&] { launch_w16_expand(ctx->stream, w, p_exp); })) return rc;
+            char xname[40];
+            snprintf(xname, sizeof xname, "%s.bf16", name);
+            if (int rc = run(ctx, xname, [&] {
+                    launch_gemm_bf16(ctx->stream, ctx->num_cu, xb, p_exp, bp, act, yp, y->dtype, rows, N, K);
+                }))
+                return rc;
+            return ok();
         }
         const int cfg = plan_gemm_w16_dma(ctx->num_cu, rows, N);
         char pname[40];  // e.g. "gemm_w16_q8.c2": the tile configuration

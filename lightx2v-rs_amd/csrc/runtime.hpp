@@ -156,13 +156,18 @@ struct lx2v_hip_ctx {
     lx2v::Stage kv_spare;  // the MemRoPE update's output layout, swapped with the cache it updates
     lx2v::Stage resid;     // linear_residual's output where the add cannot ride in the GEMM
     lx2v::Stage attn;      // split attention's partial sums (attention_split)
-    lx2v::Stage wexp;      // a Q8 / Q4 / FP8 weight's bf16 values for one call (w16_expand_chosen)
+    lx2v::Stage wexp;      // a Q8 / Q4 / FP8 weight's bf16 values for one call (plan_w16; at most 128 MB)
+    size_t wexp_refused = SIZE_MAX;  // the least size of it that the device had no room for
     lx2v::Stage splitk;    // split-K fp8 GEMM partial sums (Fp8Plan::splits)
     // The no-alloc entry point's hold on the device scratch: recorded after
     // each of its calls (and each launch of a graph that holds such calls);
     // capture_scratch: the capture in progress recorded one.
     hipEvent_t scratch_done = nullptr;
     bool capture_scratch = false;
+    // Captured graphs not yet freed, and the workspace blocks outgrown since
+    // the first of them: a replay may still use those.
+    int graphs = 0;
+    std::vector<void *> outgrown;
 };
 
 namespace lx2v {

@@ -80,3 +80,67 @@ def test_expanded_weight_equals_dequantized(be, monkeypatch, fmt, xdt, M, K, N):
             assert np.array_equal(u32(out[0]), u32(out[1]))
     finally:
         be.set_fp8_act(H.FP8_ACT_E4M3)
+
+
+def _q8(be, seed, N, K):
+    codes = (np.arange(N * K, dtype=np.uint32) * np.uint32(2654435761 + 2 * seed) >> np.uint32(24)).astype(np.uint8)
+    return be.weight_q8(codes.view(np.int8), np.full(N * K // 32, 1e-3, np.float32), N, K, 32)
+
+
+# 3 MB written out; 48 MiB and 128 KB, past the no-alloc scratch (its tiles give the same bits)
+@pytest.mark.parametrize("M,K,N", [(300, 1024, 1536), (65, 8192, 3080)])
+@pytest.mark.parametrize("xdt", [H.DTYPE_F32, H.DTYPE_BF16])
+def test_expanded_without_allocations(be, monkeypatch, xdt, M, K, N):
+    monkeypatch.setenv("LIGHTX2V_HIP_ROWS", "0")
+    monkeypatch.setenv("LIGHTX2V_HIP_W16_EXPAND", "1")
+    w, x, b = _q8(be, 1, N, K), be.alloc((M + 1) * K, xdt), be.upload(normal(4602, N, 0.01))
+    be.write(x, normal(4601, (M + 1) * K))
+    want, names = _run(be, x, w, b, H.ACT_NONE, M, N, H.DTYPE_F32)
+    assert "w16_expand" in names
+    y = be.alloc(M * N)
+    for _ in range(2):
+        be.write(y, np.full(M * N, np.nan, np.float32))
+        be.linear_noalloc(x, 1, M, w, b, H.ACT_NONE, y, 0)
+        assert np.array_equal(u32(be.download(y)), u32(want).ravel())
+
+
+def test_expanded_in_graphs(monkeypatch):
+    """A graph captured before there is a workspace for the written-out weight,
+    and one captured after; then the context's workspaces outgrow what the
+    graphs hold.  Every replay gives the eager bits, with eager work between."""
+    monkeypatch.setenv("LIGHTX2V_HIP_ROWS", "0")
+    monkeypatch.setenv("LIGHTX2V_HIP_W16_EXPAND", "1")
+    be = H.HipBackend(0)
+    try:
+        M, K, N = 300, 1024, 1536
+        w, x = _q8(be, 2, N, K), be.alloc(M * K, H.DTYPE_F32)
+        xb = be.alloc(M * K, H.DTYPE_BF16)
+        for buf in (x, xb):
+            be.write(buf, normal(4701, M * K))
+        y, y2, want = be.alloc(M * N), be.alloc(M * N), be.alloc(M * N)
+
+        def capture(src, dst):
+            be.graph_begin()
+            be.linear(src, 0, M, w, None, H.ACT_GELU_TANH, dst, 0)
+            return be.graph_end()
+
+        graphs = [capture(xb, y)]  # no workspace yet: the tiles
+        be.linear(x, 0, M, w, None, H.ACT_GELU_TANH, want, 0)
+        ref = u32(be.download(want)).copy()
+        graphs.append(capture(x, y2))
+        big, bx, by = _q8(be, 3, 4096, 2048), be.alloc(900 * 2048, H.DTYPE_F32), be.alloc(900 * 4096)
+        be.write(bx, normal(4702, 900 * 2048))
+        for rep in range(3):
+            be.linear(bx, 0, 900, big, None, H.ACT_NONE, by, 0)  # (the first of these grows both workspaces)
+            for g, dst in zip(graphs, (y, y2)):
+                be.write(dst, np.full(M * N, np.nan, np.float32))
+                be.sync()
+                g.launch()
+                be.linear(bx, 0, 300 + 300 * rep, big, None, H.ACT_NONE, by, 0)
+                assert np.array_equal(u32(be.download(dst)), ref), rep
+        for g in graphs:
+            g.free()
+        be.linear(x, 0, M, w, None, H.ACT_GELU_TANH, want, 0)
+        assert np.array_equal(u32(be.download(want)), ref)
+    finally:
+        be.close()
