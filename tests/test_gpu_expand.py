@@ -1,7 +1,7 @@
-"""Two ways to the same sums on the bf16 MFMA: the 256 x 256 persistent tile
-against the 256 x 128 one (LIGHTX2V_HIP_BF16_CFG), and a Q8 / Q4 / FP8 weight
-written out as bf16 first against dequantization inside the GEMM
-(LIGHTX2V_HIP_W16_EXPAND).  Both sides contract the same bf16 values in the
+"""Ways to the same sums on the bf16 MFMA: the tiles of the bf16 GEMM among each
+other (LIGHTX2V_HIP_BF16_CFG), and a Q8 / Q4 / FP8 weight written out as bf16
+first against dequantization inside the GEMM (LIGHTX2V_HIP_W16_EXPAND), also
+in graphs and without allocations.  All contract the same bf16 values in the
 same 16-element steps in the same order, so outputs agree bit for bit."""
 
 import numpy as np
@@ -46,6 +46,30 @@ def test_bf16_persistent_tile_equals_tiles(be, monkeypatch, act, M, K, N):
     p = np.unique(np.append(np.arange(0, M, 97), M - 1))
     ref = oracle_w16(O.bf16_round(xf).reshape(M + 1, K)[1:][p], wf.reshape(N, K), bf if M != 257 else None, act)
     assert_close(out[1][p], ref, W16_TIGHT[0] + 2.0**-8, W16_TIGHT[1] + 2.0**-7 * np.abs(ref).max(), what="vs oracle")
+
+
+# One row and around a 64-row tile, past two; K of one stage, below and past the ring's four slots
+@pytest.mark.parametrize("K", [64, 192, 320])
+@pytest.mark.parametrize("M,N", [(1, 33), (63, 128), (64, 64), (65, 130), (129, 264), (300, 513)])
+def test_bf16_tiles_agree(be, monkeypatch, M, N, K):
+    """Every one-shot tile (256 x 128, 128 x 256, 128 x 128, 64 x 128, 64 x 64)
+    against the first, bit for bit, and against the oracle."""
+    monkeypatch.setenv("LIGHTX2V_HIP_ROWS", "0")
+    wf, xf, bf = normal(4451 + N, N * K, 0.02), normal(4452 + M, (M + 1) * K), normal(4453, N, 0.01)
+    w, x, b = be.weight(wf, N, K), be.alloc((M + 1) * K, H.DTYPE_BF16), be.upload(bf)
+    be.write(x, xf)
+    ref = oracle_w16(O.bf16_round(xf).reshape(M + 1, K)[1:], wf.reshape(N, K), bf, 1)
+    for ydt in (H.DTYPE_F32, H.DTYPE_BF16):
+        out = []
+        for cfg in range(5):
+            monkeypatch.setenv("LIGHTX2V_HIP_BF16_CFG", str(cfg))
+            out.append(_run(be, x, w, b, H.ACT_GELU_TANH, M, N, ydt)[0])
+            assert np.array_equal(u32(out[0]), u32(out[-1])), (cfg, ydt)
+        if ydt == H.DTYPE_F32:
+            assert_close(out[0], ref, *W16_TIGHT, what=f"{M}x{K}->{N}")
+        else:
+            assert np.array_equal(u32(out[0]), u32(O.bf16_round(f32).reshape(M, N)))
+        f32 = out[0]
 
 
 @pytest.mark.parametrize("M,K,N", [(1, 64, 33), (300, 192, 96), (257, 1536, 512)])

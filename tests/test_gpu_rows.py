@@ -1,8 +1,9 @@
-"""The few-rows linear (csrc/k_gemm_rows.hip, up to 64 rows) against the tile
-kernels on the same operands (LIGHTX2V_HIP_ROWS=0), for every weight format and
-activation / output type that takes it, at its edges: one row, whole and
-ragged 32-row blocks, whole and ragged 32-channel blocks, K below, at and past
-the eight waves' first steps, row offsets.
+"""The few-rows linear (csrc/k_gemm_rows.hip: FP8 up to 64 rows, the others up to
+256) against the tile kernels on the same operands (LIGHTX2V_HIP_ROWS=0), for
+every weight format and activation / output type that takes it, at its edges:
+one row, whole and ragged 32-row blocks, one to four 64-row workgroups, whole
+and ragged 32-channel blocks, K below, at and past the eight waves' first
+steps, row offsets.  And which of the ways a call takes.
 
 Both sides contract the same e4m3 / bf16 operands and differ in the order of
 their f32 sums (and in the point where a group's scale enters): FP8_TIGHT
@@ -44,7 +45,7 @@ def _weight(be, fmt, N, K):
 
 
 def _linear(be, monkeypatch, few, x, row, M, w, b, act, y, y_row):
-    monkeypatch.setenv("LIGHTX2V_HIP_ROWS", "64" if few else "0")
+    monkeypatch.setenv("LIGHTX2V_HIP_ROWS", "256" if few else "0")
     be.profile_reset()
     be.profile_enable(True)
     try:
@@ -81,6 +82,29 @@ def test_rows_vs_tiles(be, monkeypatch, fmt, xdt, M, K, N):
     y16 = be.alloc(M * N, H.DTYPE_BF16)
     _linear(be, monkeypatch, True, xb, 3, M, w, bb, H.ACT_GELU_TANH, y16, 0)
     assert np.array_equal(u32(be.download(y16)), u32(O.bf16_round(out[1]).ravel()))
+
+
+@pytest.mark.parametrize("M,K,N", [(65, 1152, 33), (128, 192, 64), (129, 1536, 96), (256, 64, 1000)])
+@pytest.mark.parametrize("xdt", [H.DTYPE_F32, H.DTYPE_BF16])
+@pytest.mark.parametrize("fmt", ["native", "q8_32", "q4_32", "q4_zeros_32", "fp8_64"])
+def test_rows_past_one_workgroup(be, monkeypatch, fmt, xdt, M, K, N):
+    """More than 64 rows: workgroups of 64, the last one ragged."""
+    if fmt == "fp8_64" and K == 64:
+        pytest.skip("one group per channel: the fp8 MFMA")
+    w, wd = _weight(be, fmt, N, K)
+    x, b = normal(4401 + M, (M + 3) * K).reshape(M + 3, K), normal(4402, N, 0.01)
+    xb, bb = be.alloc(x.size, xdt), be.upload(b)
+    be.write(xb, x)
+    out = []
+    for few in (False, True):
+        y = be.alloc((M + 2) * N, H.DTYPE_F32)
+        be.write(y, np.full((M + 2) * N, np.nan, np.float32))
+        _linear(be, monkeypatch, few, xb, 3, M, w, bb, H.ACT_GELU_TANH, y, 1)
+        v = be.download(y).reshape(M + 2, N)
+        assert np.isnan(v[0]).all() and np.isnan(v[-1]).all()
+        out.append(v[1:-1])
+    assert_close(out[1], out[0], *W16_TIGHT, what=f"{fmt} rows vs tiles")
+    assert_close(out[1], oracle_w16(x[3:], wd, b, 1), *W16_TIGHT, what=f"{fmt} rows vs oracle")
 
 
 @pytest.mark.parametrize("M,K,N", [(1, 128, 32), (17, 1536, 96), (33, 1152, 64), (64, 2304, 1024)])
