@@ -140,7 +140,7 @@ def per_config(be, H):
         be.profile_enable(True)
         try:
             be.linear(x, 0, rows, w, b, act, y, 0)
-            ran = sorted(kk for kk in be.profile_stats() if kk.startswith("gemm"))
+            ran = sorted((kk for kk in be.profile_stats() if kk.startswith(("gemm", "w16_expand"))), reverse=True)
         finally:
             be.profile_enable(False)
             be.profile_reset()
@@ -164,6 +164,9 @@ def per_config(be, H):
     g128_chunk_path = ("the chunk's input as its producer writes it (per-token e4m3: QKV, cross Q, the text K/V, "
                        "FFN up; MX e4m3: O, cross O, FFN down) x FP8 weight with one scale per 128 columns, fp8 "
                        "MFMA; bf16 output (FFN up: MX e4m3)")
+    # (alg_bytes counts the stored weight only: writing its bf16 values out and reading them is the path's own traffic)
+    w16_path = ("bf16 MFMA on the weight's bf16 values, written out by a pass of their own (w16_expand in `kernel`) or "
+                "else dequantized inside the GEMM; us_per_linear holds both launches")
     # config 1: FP8 self-attn Q projection, f32 activations in and out
     be.set_act_dtype(H.DTYPE_F32)
     x = be.alloc(M * DIM)
@@ -211,7 +214,7 @@ def per_config(be, H):
     be.fill_normal(x, 1011, 1.0)
     w = weight("q8", FFN, DIM, 0.02, 1012)
     time_linear("cfg2_q8_ffn_up_gelu", x, M, DIM, w, FFN, 1, H.DTYPE_BF16, H.DTYPE_BF16, PEAK_BF16_TFLOPS,
-                "bf16 activations x Q8 weight dequantized to bf16 inside the GEMM, bf16 MFMA", kind="q8", group=32)
+                "bf16 activations x Q8 weight, " + w16_path, kind="q8", group=32)
     w.free()
     x.free()
     # config 3: Q4 (symmetric, per-32 scales) FFN down, input = GELU of N(0,1); plain and heavy-tailed
@@ -228,7 +231,7 @@ def per_config(be, H):
         w = weight("q4", DIM, FFN, 0.02, 1022, heavy=heavy)
         time_linear("cfg3_q4_ffn_down" + ("_heavy_tailed" if heavy else ""), x, M, FFN, w, DIM, 0,
                     H.DTYPE_BF16, H.DTYPE_BF16, PEAK_BF16_TFLOPS,
-                    "bf16 activations x Q4 weight dequantized to bf16 inside the GEMM, bf16 MFMA", kind="q4", group=32)
+                    "bf16 activations x Q4 weight, " + w16_path, kind="q4", group=32)
         w.free()
     x.free()
     # config 5: Wan2.2-TI2V-5B shapes in FP8, M = 2640 and 880
@@ -323,7 +326,7 @@ def yardstick(be, H):
                    "this_build_tflops": round(2.0 * rows * n * k / t_ours / 1e6, 1)}
         log(f"yardstick {nm} {rows}x{k}->{n}: hipBLASLt {t_blas:.2f} us, this build {t_ours:.2f} us")
     # bf16: hipBLASLt's GEMM (torch.mm, bf16 x bf16 -> bf16) beside this build's
-    # Q8 / Q4 linears (per-32 scales, dequantized to bf16 in the K loop) and its
+    # Q8 / Q4 linears (per-32 scales, contracted as bf16) and its
     # native bf16-weight linear at configs 2 and 3's shapes, and 8192^3
     res16 = {}
     for nm, rows, n, k, act in (("cfg2_ffn_up", M, FFN, DIM, 1), ("cfg3_ffn_down", M, DIM, FFN, 0),

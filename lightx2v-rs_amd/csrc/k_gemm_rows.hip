@@ -1,18 +1,23 @@
 // k_gemm_rows.hip -- Backend::linear over few activation rows
 // (crates/lightx2v-core/src/backend.rs:198-212): every weight format on the
 // MFMA that the tiled kernels use for it (k_gemm_fp8.hip, k_gemm_w16.hip),
-// laid out for a weight that is read once.
+// laid out for few rows beside the weight's bytes.
 //
-//   Y[m, n] = act( sum_k X[m, k] W[n, k] + bias[n] )      M <= 64 MB rows a workgroup
+//   Y[m, n] = act( sum_k X[m, k] W[n, k] + bias[n] )
+//
+// A workgroup takes 32 MB rows (MB = 1 or 2) and 32 channels: the weight is
+// read once for every 64 rows (up to 64 with FP8 weights on the fp8 MFMA, 256
+// with the others).
 //
 // What bounds it: latency and the weight's bytes.  A tile of the other
 // kernels walks all of K in one workgroup, 128 channels wide: at 17 rows,
 // 1536 -> 1536 occupies 12 CUs for 12 serial stages (8.2 us), and 1536 <-
-// 14336 for 112 (33 us).  Here a workgroup takes 32 channels and splits K over
-// its eight waves in 128-element steps (wave w: steps w, w + 8, ...).  Each
-// wave loads its operands from global memory straight into MFMA fragments,
-// two steps ahead of the one it contracts, with no LDS and no barrier; the
-// eight partial sums meet once in LDS, in wave order, and the epilogue stores.
+// 14336 for 112 (33 us).  Here a workgroup splits K over its eight waves in
+// steps of 128 elements (64 where the operands of one take more registers;
+// wave w: steps w, w + 8, ...).  Each wave loads its operands from global
+// memory straight into MFMA fragments, one or two steps ahead of the one it
+// contracts, with no LDS and no barrier; the eight partial sums meet once in
+// LDS, in wave order, and the epilogue stores (6.0 and 22 us).
 //
 // Fragments: the activations are the MFMA's A operand and the weight its B
 // operand, so a lane holds one channel (l % 32) and 16 rows, and a group's

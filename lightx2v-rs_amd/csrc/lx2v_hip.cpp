@@ -2049,7 +2049,7 @@ static int linear_run(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_row, si
     // A dequantized weight: inside the GEMM, or written out first.
     const bool w16_dma = !e4m3_path && !native_bf16 && gemm_w16_dma_supported(w, rows);
     const W16Plan w16 = w16_dma ? plan_w16(ctx->num_cu, w, rows, y->dtype) : W16Plan{};
-    // Few rows: the kernels that read the weight once, on the same operands.
+    // Few rows: the kernels laid out for them, on the same operands.
     // (Decided by shapes and types alone, so that a call gives the same bits
     // eagerly, captured and without allocations.)
     bool few = false;
@@ -2292,10 +2292,12 @@ int lx2v_hip_linear_noalloc(lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t x_r
 }
 
 // The residual add can ride in the GEMM's epilogue: FP8 weight with one scale
-// per channel on the e4m3 path, a bf16 / f32 output, and a direct-to-LDS
-// configuration (K % 128 == 0; not the 256 x 256 ping-pong tile), where
-// linear itself would not split K (its sums would then be added in another
-// order than the fused kernel's; the pair keeps the two equal).
+// per channel or per 128 columns on the e4m3 path, a bf16 / f32 output, and
+// the few-rows kernel (K % 64 == 0) or a direct-to-LDS configuration (K % 128
+// == 0; not the persistent tiles nor the ping-pong one), where linear itself
+// would take the few-rows kernel too, or would not split K (its sums would
+// then be added in another order than the fused kernel's; the pair keeps the
+// two equal).
 static bool linear_fusable(const lx2v_hip_ctx *ctx, const lx2v_hip_buf *x, size_t rows, const lx2v_hip_weight *w,
                            const lx2v_hip_buf *h, int act) {
     const size_t N = w->rows, K = w->cols;
